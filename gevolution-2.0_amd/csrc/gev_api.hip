@@ -698,11 +698,11 @@ int gev_solve_chi(gev_ctx *c, const void *Sij, void *chi, void *SijFT, void *chi
 int gev_solve_chi_Tij(gev_ctx *c, const void *phi, void *Tij, double coeff, void *chi, void *SijFT, void *chiFT)
 {
     CHECK(c && phi && Tij && chi && SijFT && chiFT, "gev_solve_chi_Tij: NULL argument");
-    if (chi_from_Tij_supported(c))
+    if (fused_sources_supported(c))
         return PREC_DISPATCH(c,
-                             solve_chi_Tij_fused_impl<double>(c, (const double *)phi, (const double *)Tij, coeff,
+                             solve_chi_Tij_fused_impl<double>(c, (const double *)phi, (double *)Tij, coeff,
                                                               (double *)chi, (cx<double> *)SijFT, (cx<double> *)chiFT),
-                             solve_chi_Tij_fused_impl<float>(c, (const float *)phi, (const float *)Tij, coeff,
+                             solve_chi_Tij_fused_impl<float>(c, (const float *)phi, (float *)Tij, coeff,
                                                              (float *)chi, (cx<float> *)SijFT, (cx<float> *)chiFT));
     // small meshes: Sij in place over Tij, then the chi solve
     int rc = gev_prepare_source_Tij(c, phi, Tij, Tij, coeff);
@@ -727,14 +727,14 @@ int gev_solve_poisson_T00(gev_ctx *c, const void *phi, const void *chi, void *so
                           double *sums)
 {
     CHECK(c && phi && chi && source && pot && work, "gev_solve_poisson_T00: NULL argument");
-    if (chi_from_Tij_supported(c)) {
+    if (fused_sources_supported(c)) {
         int rc = PREC_DISPATCH(c,
                                solve_poisson_T00_fused_impl<double>(c, (const double *)phi, (const double *)chi,
-                                                                    (const double *)source, bg, c1, c2, c3,
+                                                                    (double *)source, bg, c1, c2, c3,
                                                                     (double *)pot, (cx<double> *)work, coeff, modif,
                                                                     k0set),
                                solve_poisson_T00_fused_impl<float>(c, (const float *)phi, (const float *)chi,
-                                                                   (const float *)source, bg, c1, c2, c3,
+                                                                   (float *)source, bg, c1, c2, c3,
                                                                    (float *)pot, (cx<float> *)work, coeff, modif,
                                                                    k0set));
         if (rc || !sums) return rc;
@@ -761,7 +761,7 @@ int gev_ctx_sums(gev_ctx *c, double sums[2])
 int gev_solve_vector_T0i_links(gev_ctx *c, void *Bi, const void *phi, void *BiFT, double coeff, double modif)
 {
     CHECK(c && Bi && phi && BiFT, "gev_solve_vector_T0i_links: NULL argument");
-    if (chi_from_Tij_supported(c))
+    if (fused_sources_supported(c))
         return PREC_DISPATCH(c,
                              solve_vector_links_fused_impl<double>(c, (double *)Bi, (const double *)phi,
                                                                    (cx<double> *)BiFT, coeff, modif),

@@ -117,20 +117,20 @@ int gev_step(gev_pcls *p, const gev_fields *f, gev_step_state *st)
     if (st->gr) {
         // T00 (main.cu:622-651) and Tij (main.cu:750-758), both with the old phi,
         // in one pass over the particles (the outputs need no zeroing).  With
-        // the elliptic B on 128 <= N <= 1024 the same pass sums T0i
+        // the elliptic B on 16 <= N <= 1024 the same pass sums T0i
         // (main.cu:858) on the links into Bi, whose old B no step before the B
         // solve reads; the new phi's link factor is applied in the B solve.
-        const bool t0i_links = st->vector_elliptic && gev::chi_from_Tij_supported(c);
+        const bool t0i_links = st->vector_elliptic && gev::fused_sources_supported(c);
         if (t0i_links) RC(gev_project_T00_Tij_T0i_links(p, f->source, f->Sij, f->Bi, a, f->phi, 1.0));
         else RC(gev_project_T00_Tij(p, f->source, f->Sij, a, f->phi, 1.0, 0));
         RC(mark(c, GEV_PHASE_DEPOSIT_T00_TIJ));
         const double H = gev_hconf(a, fpg, om, ol, orad);
         // prepareFTsource (main.cu:725) and the phi solve (main.cu:742-794); the
-        // mixed form takes the k=0 mode from the FP64 sum.  For 128 <= N <= 1024
+        // mixed form takes the k=0 mode from the FP64 sum.  For 16 <= N <= 1024
         // the source is formed inside the solve's x pass and its sums stay on
         // the device until the end of the cycle (no wait here).
         bool t00_sums_pending = false;
-        if (dtau_old > 0. && gev::chi_from_Tij_supported(c)) {
+        if (dtau_old > 0. && gev::fused_sources_supported(c)) {
             RC(mark(c, GEV_PHASE_SOURCE_T00));
             RC(gev_solve_poisson_T00(c, f->phi, f->chi, f->source, om, 3. * H * dx * dx / dtau_old, fpg * dx * dx / a,
                                      3. * H * H * dx * dx, f->phi, f->scalarFT, 1. / (dx * dx), 3. * H / dtau_old,
@@ -210,9 +210,7 @@ int gev_step(gev_pcls *p, const gev_fields *f, gev_step_state *st)
     } else {
         RC(gev_project_mass(p, f->source, 1.0, 0));
         RC(mark(c, GEV_PHASE_DEPOSIT_T00_TIJ));
-        RC(gev_fft_r2c(c, f->source, f->scalarFT, 1));
-        RC(gev_poisson(c, f->scalarFT, f->scalarFT, fpg / a, 0.0)); // main.cu:765
-        RC(gev_fft_c2r(c, f->scalarFT, f->phi, 1));
+        RC(gev_solve_poisson(c, f->source, f->phi, f->scalarFT, fpg / a, 0.0, 0, 0.0)); // main.cu:742-794
         RC(mark(c, GEV_PHASE_SOLVE_PHI));
         const double a_d = gev_rk4bg(a, fpg, om, ol, orad, 0.5 * dtau);
         RC(gev_kick_drift(p, 0, (dtau + dtau_old) / 2., dtau, f->phi, nullptr, nullptr, 1, 0, a, a_d, 1.0, 1.0,

@@ -2,10 +2,14 @@
 // passes: x (real<->half-complex, contiguous lines), then y and z (complex,
 // strided columns read as TX-wide coalesced row segments).  Radix-8/4/2
 // Stockham stages in LDS, twiddles from a per-size table in global memory.
+// For 16 <= N <= 128 the x and y passes are one kernel per plane
+// (gev_fft_plane.hpp), all components of a field in one launch.
+#include <algorithm>
 #include <type_traits>
 
 #include "gev_common.hpp"
 #include "gev_fft_engine.hpp"
+#include "gev_fft_plane.hpp"
 #include "gev_kernels.hpp"
 #include "gev_kops.hpp"
 
@@ -167,7 +171,8 @@ template <typename T> constexpr int tx_of() { return sizeof(T) == 8 ? 8 : 16; }
 template <typename T, int L> constexpr int col_tx() { return (tx_of<T>() * L / 8 > 1024) ? 8192 / L : tx_of<T>(); }
 template <typename T, int N> constexpr int xlines() { return (sizeof(T) == 8 ? 4096 : 8192) / N; }
 
-// y / z column pass, in place: TX adjacent kx columns x one full line.
+// y / z column pass, in place: TX adjacent kx columns x one full line; the
+// grid covers one or several consecutive components.
 template <typename T, int L, int TX>
 __global__ __launch_bounds__(TX * L / 8) void k_col_reg(cx<T> *__restrict__ data, int P, int axis, int dir,
                                                         const cx<T> *__restrict__ tw)
@@ -175,17 +180,17 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_reg(cx<T> *__restrict__ data
     constexpr int NT = TX * L / 8;
     __shared__ cx<T> lds[TX * (L + 1)];
     __shared__ cx<T> twl[L];
-    for (int m = threadIdx.x; m < L; m += NT) twl[m] = tw[m];
+    const TwiddleLoad<T, L, NT> twload(twl, tw);
     const int ntiles = P / TX;
     const int64_t b = xcd_remap(blockIdx.x, gridDim.x);
     const int ct = (int)(b % ntiles);
     const int64_t o = b / ntiles;
     const int64_t stride = (axis == 1) ? (int64_t)P : (int64_t)P * L;
-    cx<T> *base = data + (int64_t)ct * TX + ((axis == 1) ? (int64_t)P * L * o : (int64_t)P * o);
+    cx<T> *base = data + (int64_t)ct * TX +
+                  ((axis == 1) ? (int64_t)P * L * o : (int64_t)P * ((o & (L - 1)) + (int64_t)L * L * (o / L)));
     auto ld = [&](int line, int row) { return base[(int64_t)row * stride + line]; };
     auto st = [&](int line, int row, cx<T> v, int) { base[(int64_t)row * stride + line] = v; };
-    __syncthreads();
-    reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, dir, ld, st);
+    reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, dir, ld, st, twload);
 }
 
 // Sources of the r2c x pass: the pair of reals (2n, 2n+1) of line L (= y + N z)
@@ -315,14 +320,13 @@ __global__ __launch_bounds__(NL * N / 16) void k_r2c_x_reg(Src src, cx<T> *__res
     constexpr int H = N / 2, NT = NL * H / 8, LDL = H + 1;
     __shared__ cx<T> lds[NL * LDL];
     __shared__ cx<T> twl[N];
-    for (int m = threadIdx.x; m < N; m += NT) twl[m] = tw[m];
+    const TwiddleLoad<T, N, NT> twload(twl, tw);
     const int64_t line0 = (int64_t)blockIdx.x * NL;
     Src sr = src;  // a source that sums keeps its sums per thread
     if constexpr (Src::kSums) sr.acc[0] = sr.acc[1] = 0.0;
     auto ld = [&](int line, int n) { return (line0 + line < nlines) ? sr(line0 + line, n) : mk((T)0, (T)0); };
     auto st = [&](int line, int k, cx<T> v, int) { lds[line * LDL + k] = v; };
-    __syncthreads();
-    reg_fft<T, H, NL, false, 2, true, 1>(lds, twl, -1, ld, st);
+    reg_fft<T, H, NL, false, 2, true, 1>(lds, twl, -1, ld, st, twload);
     if constexpr (Src::kSums) {
         // workgroup partials of the two sums, one slot pair per workgroup
         __shared__ double ws[NT / 64][2];
@@ -368,7 +372,7 @@ __global__ __launch_bounds__(NL * N / 16) void k_r2c_x_multi(Src src, cx<T> *__r
     constexpr int H = N / 2, NT = NL * H / 8, LDL = H + 1;
     __shared__ cx<T> lds[NL * LDL];
     __shared__ cx<T> twl[N];
-    for (int m = threadIdx.x; m < N; m += NT) twl[m] = tw[m];
+    const TwiddleLoad<T, N, NT> twload(twl, tw);
     const int64_t line0 = (int64_t)blockIdx.x * NL;
     auto comp = [&](auto cc) {
         constexpr int C = decltype(cc)::value;
@@ -376,8 +380,12 @@ __global__ __launch_bounds__(NL * N / 16) void k_r2c_x_multi(Src src, cx<T> *__r
             return (line0 + line < nlines) ? src.template get<C>(line0 + line, n) : mk((T)0, (T)0);
         };
         auto st = [&](int line, int k, cx<T> v, int) { lds[line * LDL + k] = v; };
-        __syncthreads();  // twiddles loaded; the previous component's stores have read lds
-        reg_fft<T, H, NL, false, 2, true, 1>(lds, twl, -1, ld, st);
+        if constexpr (C == 0) {
+            reg_fft<T, H, NL, false, 2, true, 1>(lds, twl, -1, ld, st, twload);
+        } else {
+            __syncthreads();  // the previous component's stores have read lds
+            reg_fft<T, H, NL, false, 2, true, 1>(lds, twl, -1, ld, st);
+        }
         __syncthreads();
         cx<T> *dst = out + C * NK + line0 * P;
         for (int e = threadIdx.x; e < NL * P; e += NT) {
@@ -434,7 +442,7 @@ __global__ __launch_bounds__(NL * N / 16) void k_c2r_x_reg(const cx<T> *__restri
     constexpr int H = N / 2, NT = NL * H / 8, LDL = H + 1;
     __shared__ cx<T> lds[NL * LDL];
     __shared__ cx<T> twl[N];
-    for (int m = threadIdx.x; m < N; m += NT) twl[m] = tw[m];
+    const TwiddleLoad<T, N, NT> twload(twl, tw);
     const int64_t line0 = (int64_t)blockIdx.x * NL;
     const cx<T> *src = in + line0 * P;
     static_assert(LDL == H + 1, "a staged line holds X[0..H]");
@@ -442,6 +450,7 @@ __global__ __launch_bounds__(NL * N / 16) void k_c2r_x_reg(const cx<T> *__restri
         const int l = e / LDL;
         lds[e] = (line0 + l < nlines) ? src[(int64_t)l * P + (e - l * LDL)] : mk((T)0, (T)0);
     }
+    twload();
     __syncthreads();
     auto ld = [&](int line, int k) {
         const cx<T> *row = lds + line * LDL;
@@ -478,10 +487,11 @@ static void launch_r2c_src(const Src &src, cx<T> *out, int P, int64_t nlines, co
 template <typename T, int N>
 static void launch_r2c(const T *in, cx<T> *out, int P, int64_t nlines, const cx<T> *tw, hipStream_t s)
 {
-    if constexpr (N >= 128) {
+    if constexpr (N >= 256) {
         launch_r2c_src<T, N>(SrcPlain<T, N>{in}, out, P, nlines, tw, s);
     } else {
-        constexpr int NLINES = (4096 / N > 1024) ? 1024 : 4096 / N;
+        static_assert(N <= 8, "16 <= N <= 128 transforms whole planes");
+        constexpr int NLINES = 4096 / N > 1024 ? 1024 : 4096 / N;
         int64_t nb = (nlines + NLINES - 1) / NLINES;
         hipLaunchKernelGGL((k_r2c_x<T, N, NLINES>), dim3((unsigned)nb), dim3(FFT_NT), 0, s, in, out, P, nlines, tw);
     }
@@ -490,53 +500,102 @@ static void launch_r2c(const T *in, cx<T> *out, int P, int64_t nlines, const cx<
 template <typename T, int N>
 static void launch_c2r(const cx<T> *in, T *out, int P, int64_t nlines, const cx<T> *tw, hipStream_t s)
 {
-    if constexpr (N >= 128) {
+    if constexpr (N >= 256) {
         constexpr int NL = xlines<T, N>();
         int64_t nb = (nlines + NL - 1) / NL;
         hipLaunchKernelGGL((k_c2r_x_reg<T, N, NL>), dim3((unsigned)nb), dim3(NL * N / 16), 0, s, in, out, P, nlines,
                            tw);
     } else {
-        constexpr int NLINES = (4096 / N > 1024) ? 1024 : 4096 / N;
+        static_assert(N <= 8, "16 <= N <= 128 transforms whole planes");
+        constexpr int NLINES = 4096 / N > 1024 ? 1024 : 4096 / N;
         int64_t nb = (nlines + NLINES - 1) / NLINES;
         hipLaunchKernelGGL((k_c2r_x<T, N, NLINES>), dim3((unsigned)nb), dim3(FFT_NT), 0, s, in, out, P, nlines, tw);
     }
 }
 
+// axis 1 (y) or 2 (z) of ncomp consecutive components
 template <typename T, int N>
-static void launch_col(cx<T> *data, int P, int axis, int dir, const cx<T> *tw, hipStream_t s)
+static void launch_col(cx<T> *data, int P, int axis, int dir, const cx<T> *tw, hipStream_t s, int ncomp = 1)
 {
-    if constexpr (N >= 64) {
+    if constexpr (N >= 16) {
         constexpr int TX = col_tx<T, N>();
-        int64_t nb = (int64_t)(P / TX) * N;
+        int64_t nb = (int64_t)(P / TX) * N * ncomp;
         hipLaunchKernelGGL((k_col_reg<T, N, TX>), dim3((unsigned)nb), dim3(TX * N / 8), 0, s, data, P, axis, dir, tw);
     } else {
         constexpr int TX = tx_of<T>();
         int64_t nb = (int64_t)(P / TX) * N;
-        hipLaunchKernelGGL((k_c2c_col<T, N, TX>), dim3((unsigned)nb), dim3(FFT_NT), 0, s, data, P, axis, dir, tw);
+        for (int c = 0; c < ncomp; c++)
+            hipLaunchKernelGGL((k_c2c_col<T, N, TX>), dim3((unsigned)nb), dim3(FFT_NT), 0, s,
+                               data + (int64_t)c * P * N * N, P, axis, dir, tw);
     }
 }
 
-#define GEV_FOR_EACH_N(X) X(4) X(8) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+// the sources of the plane transforms' components (k_fwd_plane)
+template <typename T, int N> struct CompPlain {
+    const T *in;
+    int64_t M;
+    template <class F> __device__ __forceinline__ void with(int c, F f) const { f(SrcPlain<T, N>{in + c * M}); }
+};
+
+constexpr bool plane_size(int N) { return N >= 16 && N <= 128; }
+
+// forward x and y passes of ncomp components (r2c without the z pass) from
+// plane sources, and the inverse y and x passes
+template <typename T, int N, class Comp>
+static void launch_fwd_plane(gev_ctx *c, const Comp &comp, cx<T> *out, int ncomp, const cx<T> *tw,
+                             double *partials = nullptr)
+{
+    hipLaunchKernelGGL((k_fwd_plane<T, N, Comp>), dim3(N / plane_np<N>(), ncomp), dim3(plane_nt<N>()), 0, c->stream,
+                       comp, out, c->NK, tw, partials);
+}
+template <typename T, int N> static void fwd_xy(gev_ctx *c, const T *in, cx<T> *out, int ncomp, const cx<T> *tw)
+{
+    if constexpr (plane_size(N)) {
+        launch_fwd_plane<T, N>(c, CompPlain<T, N>{in, c->M}, out, ncomp, tw);
+    } else {
+        for (int i = 0; i < ncomp; i++) {
+            launch_r2c<T, N>(in + i * c->M, out + i * c->NK, c->P, (int64_t)N * N, tw, c->stream);
+            launch_col<T, N>(out + i * c->NK, c->P, 1, -1, tw, c->stream);
+        }
+    }
+}
+template <typename T, int N> static void inv_yx(gev_ctx *c, cx<T> *in, T *out, int ncomp, const cx<T> *tw)
+{
+    if constexpr (plane_size(N)) {
+        hipLaunchKernelGGL((k_inv_plane<T, N>), dim3(N / plane_np<N>(), ncomp), dim3(plane_nt<N>()), 0, c->stream, in,
+                           out, c->NK, c->M, tw);
+    } else {
+        for (int i = 0; i < ncomp; i++) {
+            launch_col<T, N>(in + i * c->NK, c->P, 1, +1, tw, c->stream);
+            launch_c2r<T, N>(in + i * c->NK, out + i * c->M, c->P, (int64_t)N * N, tw, c->stream);
+        }
+    }
+}
+
+#define GEV_FOR_FUSED_N(X) X(16) X(32) X(64) X(128) X(256) X(512) X(1024)
+#define GEV_FOR_EACH_N(X) X(4) X(8) GEV_FOR_FUSED_N(X)
+
+// components at a time: all of them where a component is small (launches and
+// latency count); one by one on large meshes, whose passes then find the
+// component just written in the Infinity Cache
+template <int N> constexpr int fft_batch() { return plane_size(N) ? 64 : 1; }
 
 template <typename T>
 int fft_r2c_impl(gev_ctx *ctx, const T *in, cx<T> *out, int ncomp, const cx<T> *tw)
 {
-    const int N = ctx->N, P = ctx->P;
-    const int64_t M = ctx->M, NK = ctx->NK, nlines = (int64_t)N * N;
-    for (int c = 0; c < ncomp; c++) {
-        const T *ic = in + c * M;
-        cx<T> *oc = out + c * NK;
-        switch (N) {
-#define X(n)                                                          \
-    case n:                                                           \
-        launch_r2c<T, n>(ic, oc, P, nlines, tw, ctx->stream);         \
-        launch_col<T, n>(oc, P, 1, -1, tw, ctx->stream);              \
-        launch_col<T, n>(oc, P, 2, -1, tw, ctx->stream);              \
+    const int64_t M = ctx->M, NK = ctx->NK;
+    switch (ctx->N) {
+#define X(n)                                                                        \
+    case n:                                                                         \
+        for (int c = 0; c < ncomp; c += fft_batch<n>()) {                           \
+            const int m = std::min(ncomp - c, fft_batch<n>());                      \
+            fwd_xy<T, n>(ctx, in + c * M, out + c * NK, m, tw);                     \
+            launch_col<T, n>(out + c * NK, ctx->P, 2, -1, tw, ctx->stream, m);      \
+        }                                                                           \
         break;
-            GEV_FOR_EACH_N(X)
+        GEV_FOR_EACH_N(X)
 #undef X
-        default: gev_set_error("unsupported N"); return GEV_ERR_ARG;
-        }
+    default: gev_set_error("unsupported N"); return GEV_ERR_ARG;
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
@@ -545,22 +604,19 @@ int fft_r2c_impl(gev_ctx *ctx, const T *in, cx<T> *out, int ncomp, const cx<T> *
 template <typename T>
 int fft_c2r_impl(gev_ctx *ctx, cx<T> *in, T *out, int ncomp, const cx<T> *tw)
 {
-    const int N = ctx->N, P = ctx->P;
-    const int64_t M = ctx->M, NK = ctx->NK, nlines = (int64_t)N * N;
-    for (int c = 0; c < ncomp; c++) {
-        cx<T> *ic = in + c * NK;
-        T *oc = out + c * M;
-        switch (N) {
-#define X(n)                                                          \
-    case n:                                                           \
-        launch_col<T, n>(ic, P, 2, +1, tw, ctx->stream);              \
-        launch_col<T, n>(ic, P, 1, +1, tw, ctx->stream);              \
-        launch_c2r<T, n>(ic, oc, P, nlines, tw, ctx->stream);         \
+    const int64_t M = ctx->M, NK = ctx->NK;
+    switch (ctx->N) {
+#define X(n)                                                                        \
+    case n:                                                                         \
+        for (int c = 0; c < ncomp; c += fft_batch<n>()) {                           \
+            const int m = std::min(ncomp - c, fft_batch<n>());                      \
+            launch_col<T, n>(in + c * NK, ctx->P, 2, +1, tw, ctx->stream, m);       \
+            inv_yx<T, n>(ctx, in + c * NK, out + c * M, m, tw);                     \
+        }                                                                           \
         break;
-            GEV_FOR_EACH_N(X)
+        GEV_FOR_EACH_N(X)
 #undef X
-        default: gev_set_error("unsupported N"); return GEV_ERR_ARG;
-        }
+    default: gev_set_error("unsupported N"); return GEV_ERR_ARG;
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
@@ -573,8 +629,13 @@ int fft_c2r_impl(gev_ctx *ctx, cx<T> *in, T *out, int ncomp, const cx<T> *tw)
 // every mode is read once and written once instead of three times each.
 // In place (in == out) is allowed: a workgroup reads all its columns before
 // writing them and no two workgroups share a column.
-// ZOP_SCALAR3: projectFTscalar from the three groups A, B, C that k_col_comb
-// forms in the y pass (below) instead of the six Sij components
+// ZOP_SCALAR: projectFTscalar, every weight of which is linear in the kz
+// factors g2 = gk2[kz] and k2 = ks[kz], so three combinations of the six Sij
+// components carry it through the z transform:
+//   A = (g1 - 2 g0) S_xx - 6 k0 k1 S_xy + (g0 - 2 g1) S_yy + (g0 + g1) S_zz
+//   B = S_xx + S_yy - 2 S_zz,   C = -6 (k0 S_xz + k1 S_yz)
+// ZOP_SCALAR3: the same from the three groups that k_col_comb forms in the y
+// pass (below) instead of the six components
 enum { ZOP_POISSON = 0, ZOP_SCALAR = 1, ZOP_VECTOR = 2, ZOP_SCALAR3 = 3 };
 
 struct ZParams {
@@ -583,7 +644,12 @@ struct ZParams {
     double coeff, modif;  // Poisson: coeff pre-scaled by -1/N^3; vector: as projectFTvector
     double k0re, k0im;    // Poisson: value taken for the k=0 mode when k0set
     int k0set;
-    const double *k0dev;  // when set, the real part of that mode is read here instead
+    // Poisson with the source formed in the x pass: the pass's workgroup sums
+    // (nparts pairs), reduced by the workgroup that holds the k=0 mode into
+    // sums[0], sums[1]; the real part of that mode is then sums[1] when k0set
+    const double *parts;
+    int nparts;
+    double *sums;
 };
 
 // ============================ y pass of Sij forming the groups of the z solve ==
@@ -607,11 +673,13 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int
     // the k tables in the transform's precision (the weights are applied in it)
     __shared__ T gkl[L];
     __shared__ cx<T> ksl[L];
-    for (int m = threadIdx.x; m < L; m += NT) {
-        twl[m] = tw[m];
-        gkl[m] = (T)gk2[m];
-        ksl[m] = mk((T)ks[m].x, (T)ks[m].y);
-    }
+    auto tables = [&]() {
+        for (int m = threadIdx.x; m < L; m += NT) {
+            twl[m] = tw[m];
+            gkl[m] = (T)gk2[m];
+            ksl[m] = mk((T)ks[m].x, (T)ks[m].y);
+        }
+    };
     const int ntiles = P / TX;
     const int64_t b = xcd_remap(blockIdx.x, gridDim.x);
     const int ct = (int)(b % ntiles);
@@ -637,8 +705,12 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int
             if constexpr (c == 0) rows[slot] = row;
             v[slot] = val;
         };
-        __syncthreads();  // tables loaded; the previous transform is done with lds
-        reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
+        if constexpr (c == 0) {
+            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st, tables);
+        } else {
+            __syncthreads();  // the previous transform is done with lds
+            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
+        }
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int row = rows[s];
@@ -692,29 +764,19 @@ static void launch_col_comb(cx<T> *data, int P, int64_t NK, const cx<T> *tw, con
 }
 
 // FP32 vector projection from L = 128 up: 4 waves per SIMD (two workgroups
-// per CU) at the price of a spill of up to 80 bytes, 4.5 -> 4.1 ms for the
+// per CU) at the price of a spill of up to 56 bytes, 4.5 -> 4.1 ms for the
 // 512^3 B solve; the scalar projection and FP64 measured no better that way
-// ZS2_DIRECT: the vector solve reads each component in its transform's first
-// stage and applies the projection per mode with the last one (1.31 against
-// 1.34 ms at 512^3, spill 56 against 80 bytes); 0 keeps the all-operands-first form
-#ifndef ZS2_DIRECT
-#define ZS2_DIRECT 1
-#endif
-#ifndef ZS2_WAVES
-#define ZS2_WAVES 4
-#endif
-template <typename T, int L, int OP> constexpr int zs_waves() { return (OP == 2 && sizeof(T) == 4 && L >= 128) ? ZS2_WAVES : 1; }
+template <typename T, int L, int OP> constexpr int zs_waves() { return (OP == ZOP_VECTOR && sizeof(T) == 4 && L >= 128) ? 4 : 1; }
 
 template <typename T, int L, int TX, int OP>
 __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(const cx<T> *in, cx<T> *out, int P, int64_t NK,
                                                        const cx<T> *__restrict__ tw, ZParams zp)
 {
-    constexpr int NT = TX * L / 8, LDL = L + 1;
-    constexpr int NOUT = OP == ZOP_VECTOR ? 3 : 1;
-    constexpr int NV = OP == ZOP_VECTOR ? 3 : 1;  // inputs held at once
+    constexpr int NT = TX * L / 8, LDL = L + 1, NW = (NT + 63) / 64;
+    constexpr int NV = OP == ZOP_VECTOR ? 3 : 1;  // values per mode held at once
     __shared__ cx<T> lds[TX * LDL];
     __shared__ cx<T> twl[L];
-    for (int m = threadIdx.x; m < L; m += NT) twl[m] = tw[m];
+    const TwiddleLoad<T, L, NT> twload(twl, tw);
     const int ntiles = P / TX;
     const int64_t b = xcd_remap(blockIdx.x, gridDim.x);
     const int ct = (int)(b % ntiles);
@@ -724,53 +786,127 @@ __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(c
     const int H = L / 2;
     int lines[8], poss[8];
     cx<T> vin[NV][8];
-    cx<double> acc[8];
-#pragma unroll
-    for (int s = 0; s < 8; s++) acc[s] = mk(0.0, 0.0);
     const double gy = zp.gk2[ky];
     const cx<double> kyv = zp.ks[ky];
-    // forward z transform of input component c (a compile-time index when the
-    // operator holds all inputs at once, so they stay in registers)
-    auto forward = [&](int c, auto held) {
-        constexpr int CH = decltype(held)::value;
+    __shared__ double k0src;  // the k=0 value summed here (Poisson)
+    if constexpr (OP == ZOP_POISSON) {
+        if (zp.parts && ct == 0 && ky == 0) {
+            // fixed order: per thread, per wave, then the waves in turn
+            __shared__ double ws[NW][2];
+            double v0 = 0.0, v1 = 0.0;
+            for (int j = threadIdx.x; j < zp.nparts; j += NT) {
+                v0 += zp.parts[2 * j];
+                v1 += zp.parts[2 * j + 1];
+            }
+            for (int o = NT < 64 ? NT / 2 : 32; o > 0; o >>= 1) {
+                v0 += __shfl_xor(v0, o, 64);
+                v1 += __shfl_xor(v1, o, 64);
+            }
+            if ((threadIdx.x & 63) == 0) { ws[threadIdx.x >> 6][0] = v0; ws[threadIdx.x >> 6][1] = v1; }
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                double t0 = 0.0, t1 = 0.0;
+                for (int w = 0; w < NW; w++) { t0 += ws[w][0]; t1 += ws[w][1]; }
+                zp.sums[0] = t0;
+                zp.sums[1] = t1;
+                k0src = t1;
+            }
+        }
+    }
+    // forward z transform of component c, read by the transform's first stage
+    // straight from memory; every output mode goes to st(line, kz, value, slot)
+    auto forward = [&](auto comp, auto &st) {
+        constexpr int c = decltype(comp)::value;
         const cx<T> *src = in + c * NK + off;
         auto ld = [&](int line, int row) { return src[(int64_t)row * stride + line]; };
-        auto st = [&](int line, int row, cx<T> v, int slot) {
-            lines[slot] = line;
-            poss[slot] = row;
-            if constexpr (OP == ZOP_SCALAR) {
-                const int kx = ct * TX + line;
-                if (kx <= H) {
-                    const cx<double> w =
-                        kop_scalar_weight(c, zp.gk2[kx], gy, zp.gk2[row], zp.ks[kx], kyv, zp.ks[row]);
-                    acc[slot] = acc[slot] + w * mk((double)v.x, (double)v.y);
-                }
-            } else {
-                vin[CH][slot] = v;
-            }
-        };
-        __syncthreads();  // twiddles loaded; previous transform done with lds
-        reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
+        if constexpr (c == 0) {
+            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st, twload);
+        } else {
+            __syncthreads();  // previous transform done with lds
+            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
+        }
     };
-    // ZOP_SCALAR3: the k tables in LDS (FP64), read per mode by the
-    // combination and the operator
-    constexpr bool TAB = OP == ZOP_SCALAR3;
-    __shared__ double gkd[TAB ? L : 1];
-    __shared__ cx<double> ksd[TAB ? L : 1];
-    if constexpr (TAB)
+    // inverse z transform of component j of the output from vin[held]
+    auto inverse = [&](int j, auto held) {
+        constexpr int CH = decltype(held)::value;
+        __syncthreads();  // previous transform done with lds
+#pragma unroll
+        for (int s = 0; s < 8; s++) lds[lines[s] * LDL + poss[s]] = vin[CH][s];
+        __syncthreads();
+        cx<T> *dst = out + j * NK + off;
+        auto ld2 = [&](int line, int row) { return lds[line * LDL + row]; };
+        auto st2 = [&](int line, int row, cx<T> v, int) { dst[(int64_t)row * stride + line] = v; };
+        reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, +1, ld2, st2);
+    };
+    if constexpr (OP == ZOP_POISSON) {
+        auto st = [&](int ln, int row, cx<T> v, int slot) {
+            lines[slot] = ln;
+            poss[slot] = row;
+            vin[0][slot] = v;
+        };
+        forward(std::integral_constant<int, 0>{}, st);
+#pragma unroll
+        for (int s = 0; s < 8; s++) {
+            const int kx = ct * TX + lines[s], kz = poss[s];
+            const bool zero_mode = (kx == 0 && ky == 0 && kz == 0);
+            cx<double> r = mk(0.0, 0.0);
+            if (kx <= H) {
+                cx<double> sv = mk((double)vin[0][s].x, (double)vin[0][s].y);
+                if (zero_mode && zp.k0set) sv = mk(zp.parts ? k0src : zp.k0re, zp.k0im);
+                if (!(zero_mode && zp.modif == 0.0))
+                    r = kop_poisson(sv, zp.gk2[kx] + gy + zp.gk2[kz], zp.coeff, zp.modif);
+            }
+            vin[0][s] = mk((T)r.x, (T)r.y);
+        }
+        inverse(0, std::integral_constant<int, 0>{});
+    } else if constexpr (OP == ZOP_VECTOR) {
+        // the projection applied per mode when the last component arrives, so
+        // no operator loop holds eight modes' FP64 values (1.31 against
+        // 1.34 ms at 512^3 for loading all operands first, spill 56 against 80)
+        auto fwd = [&](auto held) {
+            constexpr int CH = decltype(held)::value;
+            auto st = [&](int ln, int row, cx<T> v, int slot) {
+                lines[slot] = ln;
+                poss[slot] = row;
+                if constexpr (CH < 2) {
+                    vin[CH][slot] = v;
+                } else {
+                    const int kx = ct * TX + ln;
+                    cx<double> bo[3] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
+                    if (kx <= H && !(kx == 0 && ky == 0 && row == 0)) {
+                        const cx<double> sv[3] = {mk((double)vin[0][slot].x, (double)vin[0][slot].y),
+                                                  mk((double)vin[1][slot].x, (double)vin[1][slot].y),
+                                                  mk((double)v.x, (double)v.y)};
+                        kop_vector(sv, zp.gk2[kx] + gy + zp.gk2[row], zp.ks[kx], kyv, zp.ks[row], zp.coeff, zp.modif,
+                                   bo);
+                    }
+#pragma unroll
+                    for (int j = 0; j < 3; j++) vin[j][slot] = mk((T)bo[j].x, (T)bo[j].y);
+                }
+            };
+            forward(held, st);
+        };
+        fwd(std::integral_constant<int, 0>{});
+        fwd(std::integral_constant<int, 1>{});
+        fwd(std::integral_constant<int, 2>{});
+        inverse(0, std::integral_constant<int, 0>{});
+        inverse(1, std::integral_constant<int, 1>{});
+        inverse(2, std::integral_constant<int, 2>{});
+    } else {
+        // chi = sum_c w_c S_c from the three kz groups:
+        //   sum_c w_c S_c = FFT_z(A) + g2 FFT_z(B) + k2 FFT_z(C)
+        // so only the FP64 sums stay live between the transforms.  The k
+        // tables are read per mode from LDS (FP64).
+        __shared__ double gkd[L];
+        __shared__ cx<double> ksd[L];
         for (int m = threadIdx.x; m < L; m += NT) {
             gkd[m] = zp.gk2[m];
             ksd[m] = zp.ks[m];
         }
-    if constexpr (OP == ZOP_SCALAR3) {
-        // chi from the three kz groups (formed by the y pass):
-        //   sum_c w_c S_c = FFT_z(A) + g2 FFT_z(B) + k2 FFT_z(C)
-        // each group read by its transform's first stage straight from
-        // memory, so only the FP64 sums stay live between the transforms
-        auto fft = [&](auto kind) {
+        if constexpr (OP == ZOP_SCALAR) __syncthreads();  // read by the first loads
+        cx<double> acc[8];
+        auto group = [&](auto kind) {
             constexpr int K = decltype(kind)::value;
-            const cx<T> *src = in + K * NK + off;
-            auto ld = [&](int line, int row) { return src[(int64_t)row * stride + line]; };
             auto st = [&](int ln, int row, cx<T> v, int slot) {
                 lines[slot] = ln;
                 poss[slot] = row;
@@ -791,168 +927,39 @@ __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(c
                     vin[0][slot] = mk((T)r.x, (T)r.y);
                 }
             };
-            __syncthreads();  // tables loaded; previous transform done with lds
-            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
-        };
-        fft(std::integral_constant<int, 0>{});
-        fft(std::integral_constant<int, 1>{});
-        fft(std::integral_constant<int, 2>{});
-    } else if constexpr (OP == ZOP_VECTOR && ZS2_DIRECT) {
-        // each component read by its transform's first stage straight from
-        // memory; the projection applied per mode when the last component
-        // arrives, so no operator loop holds eight modes' FP64 values
-        auto fwd = [&](auto held) {
-            constexpr int CH = decltype(held)::value;
-            const cx<T> *src = in + CH * NK + off;
-            auto ld = [&](int line, int row) { return src[(int64_t)row * stride + line]; };
-            auto st = [&](int ln, int row, cx<T> v, int slot) {
-                lines[slot] = ln;
-                poss[slot] = row;
-                if constexpr (CH < 2) {
-                    vin[CH][slot] = v;
+            if constexpr (OP == ZOP_SCALAR3) {
+                forward(kind, st);
+            } else {
+                // from the six components, each group formed in the loads of
+                // its transform (the formulas of k_col_comb)
+                const cx<T> *src = in + off;
+                auto ld = [&](int line, int row) {
+                    const int kx = ct * TX + line;
+                    const bool valid = kx <= H;  // padding columns give 0 above
+                    const cx<T> *e = src + (int64_t)row * stride + line;
+                    const T g0 = valid ? (T)gkd[kx] : (T)0, g1 = (T)gy;
+                    const cx<T> k0 = valid ? mk((T)ksd[kx].x, (T)ksd[kx].y) : mk((T)0, (T)0);
+                    const cx<T> k1 = mk((T)kyv.x, (T)kyv.y);
+                    if constexpr (K == 0)
+                        return e[0] * (g1 - (T)2 * g0) + ((k0 * (T)-6) * k1) * e[NK] + e[3 * NK] * (g0 - (T)2 * g1) +
+                               e[5 * NK] * (g0 + g1);
+                    else if constexpr (K == 1)
+                        return e[0] + e[3 * NK] - e[5 * NK] * (T)2;
+                    else
+                        return (k0 * (T)-6) * e[2 * NK] + (k1 * (T)-6) * e[4 * NK];
+                };
+                if constexpr (K == 0) {
+                    reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st, twload);
                 } else {
-                    const int kx = ct * TX + ln;
-                    cx<double> bo[3] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
-                    if (kx <= H && !(kx == 0 && ky == 0 && row == 0)) {
-                        const cx<double> sv[3] = {mk((double)vin[0][slot].x, (double)vin[0][slot].y),
-                                                  mk((double)vin[1][slot].x, (double)vin[1][slot].y),
-                                                  mk((double)v.x, (double)v.y)};
-                        kop_vector(sv, zp.gk2[kx] + gy + zp.gk2[row], zp.ks[kx], kyv, zp.ks[row], zp.coeff, zp.modif,
-                                   bo);
-                    }
-#pragma unroll
-                    for (int j = 0; j < 3; j++) vin[j][slot] = mk((T)bo[j].x, (T)bo[j].y);
+                    __syncthreads();  // previous transform done with lds
+                    reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
                 }
-            };
-            __syncthreads();  // twiddles loaded; previous transform done with lds
-            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
-        };
-        fwd(std::integral_constant<int, 0>{});
-        fwd(std::integral_constant<int, 1>{});
-        fwd(std::integral_constant<int, 2>{});
-    } else if constexpr (OP == ZOP_VECTOR) {
-        // all 24 first-stage operands (3 components x the 8 elements reg_fft's
-        // first stage reads: line t % TX, rows t / TX + r L/8) are loaded
-        // before the first transform
-        constexpr int NB = L / 8;
-        const int line = threadIdx.x % TX, jt = threadIdx.x / TX;
-        cx<T> pre[3][8];
-#pragma unroll
-        for (int c = 0; c < 3; c++)
-#pragma unroll
-            for (int r = 0; r < 8; r++) pre[c][r] = in[c * NK + off + (int64_t)(jt + r * NB) * stride + line];
-        auto fwd = [&](auto held) {
-            constexpr int CH = decltype(held)::value;
-            auto ld = [&](int, int row) { return pre[CH][(row - jt) / NB]; };
-            auto st = [&](int ln, int row, cx<T> v, int slot) {
-                lines[slot] = ln;
-                poss[slot] = row;
-                vin[CH][slot] = v;
-            };
-            __syncthreads();  // twiddles loaded; previous transform done with lds
-            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
-        };
-        fwd(std::integral_constant<int, 0>{});
-        fwd(std::integral_constant<int, 1>{});
-        fwd(std::integral_constant<int, 2>{});
-    } else if constexpr (OP == ZOP_POISSON) {
-        forward(0, std::integral_constant<int, 0>{});
-    } else {
-        // projectFTscalar: chi = sum_c w_c S_c, and every w_c is linear in the
-        // kz factors g2 = gk2[kz] and k2 = ks[kz]; three combinations formed
-        // before the z transform carry the whole projection:
-        //   A = (g1 - 2 g0) S_xx - 6 k0 k1 S_xy + (g0 - 2 g1) S_yy + (g0 + g1) S_zz
-        //   B = S_xx + S_yy - 2 S_zz,   C = -6 (k0 S_xz + k1 S_yz)
-        //   sum_c w_c S_c = FFT_z(A) + g2 FFT_z(B) + k2 FFT_z(C)
-        // Each thread combines the 8 elements reg_fft's first stage reads
-        // (line t % TX, rows t / TX + r L/8).
-        constexpr int NB = L / 8;
-        const int line = threadIdx.x % TX, jt = threadIdx.x / TX;
-        const int kx = ct * TX + line;
-        const bool valid = kx <= H;  // padding columns give 0 below
-        const double g0 = valid ? zp.gk2[kx] : 0.0;
-        const cx<double> k0 = valid ? zp.ks[kx] : mk(0.0, 0.0);
-        const cx<double> k01 = (k0 * kyv) * -6.0, k0m = k0 * -6.0, k1m = kyv * -6.0;
-        const T wa0 = (T)(gy - 2.0 * g0), wa3 = (T)(g0 - 2.0 * gy), wa5 = (T)(g0 + gy);
-        const cx<T> wa1 = mk((T)k01.x, (T)k01.y), wc2 = mk((T)k0m.x, (T)k0m.y), wc4 = mk((T)k1m.x, (T)k1m.y);
-        cx<T> A[8], B[8], C[8];
-        const cx<T> *src = in + off + line;
-#pragma unroll
-        for (int r = 0; r < 8; r++) {
-            const int64_t e = (int64_t)(jt + r * NB) * stride;
-            const cx<T> s0 = src[e], s1 = src[NK + e], s2 = src[2 * NK + e], s3 = src[3 * NK + e],
-                        s4 = src[4 * NK + e], s5 = src[5 * NK + e];
-            A[r] = s0 * wa0 + wa1 * s1 + s3 * wa3 + s5 * wa5;
-            B[r] = s0 + s3 - s5 * (T)2;
-            C[r] = wc2 * s2 + wc4 * s4;
-        }
-        auto fft = [&](const cx<T> *pre, auto kind) {
-            constexpr int K = decltype(kind)::value;
-            auto ld = [&](int, int row) { return pre[(row - jt) / NB]; };
-            auto st = [&](int ln, int row, cx<T> v, int slot) {
-                lines[slot] = ln;
-                poss[slot] = row;
-                const cx<double> d = mk((double)v.x, (double)v.y);
-                if constexpr (K == 0) acc[slot] = d;
-                else if constexpr (K == 1) acc[slot] = acc[slot] + d * zp.gk2[row];
-                else acc[slot] = acc[slot] + zp.ks[row] * d;
-            };
-            __syncthreads();  // twiddles loaded; previous transform done with lds
-            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st);
-        };
-        fft(A, std::integral_constant<int, 0>{});
-        fft(B, std::integral_constant<int, 1>{});
-        fft(C, std::integral_constant<int, 2>{});
-    }
-    // the operator, per owned mode; the outputs replace the inputs in vin
-#pragma unroll
-    for (int s = 0; s < 8; s++) {
-        const int kx = ct * TX + lines[s], kz = poss[s];
-        const bool pad = kx > H;
-        const bool zero_mode = (kx == 0 && ky == 0 && kz == 0);
-        const double kk = (pad || TAB) ? 1.0 : zp.gk2[kx] + gy + zp.gk2[kz];
-        if constexpr (OP == ZOP_POISSON) {
-            cx<double> r = mk(0.0, 0.0);
-            if (!pad) {
-                cx<double> sv = mk((double)vin[0][s].x, (double)vin[0][s].y);
-                if (zero_mode && zp.k0set) sv = mk(zp.k0dev ? *zp.k0dev : zp.k0re, zp.k0im);
-                if (!(zero_mode && zp.modif == 0.0)) r = kop_poisson(sv, kk, zp.coeff, zp.modif);
             }
-            vin[0][s] = mk((T)r.x, (T)r.y);
-        } else if constexpr (OP == ZOP_SCALAR3) {
-            // applied with the last forward transform
-        } else if constexpr (OP == ZOP_SCALAR) {
-            cx<double> r = mk(0.0, 0.0);
-            if (!pad && !zero_mode) r = acc[s] * kop_scalar_norm(kk, L);
-            vin[0][s] = mk((T)r.x, (T)r.y);
-        } else if constexpr (!ZS2_DIRECT) {
-            cx<double> bo[3] = {mk(0.0, 0.0), mk(0.0, 0.0), mk(0.0, 0.0)};
-            if (!pad && !zero_mode) {
-                const cx<double> sv[3] = {mk((double)vin[0][s].x, (double)vin[0][s].y),
-                                          mk((double)vin[1][s].x, (double)vin[1][s].y),
-                                          mk((double)vin[2][s].x, (double)vin[2][s].y)};
-                kop_vector(sv, kk, zp.ks[kx], kyv, zp.ks[kz], zp.coeff, zp.modif, bo);
-            }
-#pragma unroll
-            for (int j = 0; j < 3; j++) vin[j][s] = mk((T)bo[j].x, (T)bo[j].y);
-        }
-    }
-    // inverse z transform of output component j
-    auto inverse = [&](int j, auto held) {
-        constexpr int CH = decltype(held)::value;
-        __syncthreads();  // previous transform done with lds
-#pragma unroll
-        for (int s = 0; s < 8; s++) lds[lines[s] * LDL + poss[s]] = vin[CH][s];
-        __syncthreads();
-        cx<T> *dst = out + j * NK + off;
-        auto ld2 = [&](int line, int row) { return lds[line * LDL + row]; };
-        auto st2 = [&](int line, int row, cx<T> v, int) { dst[(int64_t)row * stride + line] = v; };
-        reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, +1, ld2, st2);
-    };
-    inverse(0, std::integral_constant<int, 0>{});
-    if constexpr (NOUT == 3) {
-        inverse(1, std::integral_constant<int, 1>{});
-        inverse(2, std::integral_constant<int, 2>{});
+        };
+        group(std::integral_constant<int, 0>{});
+        group(std::integral_constant<int, 1>{});
+        group(std::integral_constant<int, 2>{});
+        inverse(0, std::integral_constant<int, 0>{});
     }
 }
 
@@ -963,17 +970,11 @@ __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(c
 // scalar one (150+ registers, one 512-thread workgroup per CU) runs three
 // 256-thread workgroups per CU (0.90 against 1.02 ms at 512^3, FP32); the
 // vector one measured slower that way (1.75 against 1.34 ms)
-#ifndef ZS3_THREADS
-#define ZS3_THREADS 256
-#endif
-#ifndef ZS2_THREADS
-#define ZS2_THREADS 512
-#endif
 template <typename T, int L, int OP> constexpr int zs_tx()
 {
     constexpr bool narrow = OP != ZOP_POISSON || L <= 512;
     constexpr int tx = (narrow && col_tx<T, L>() * L / 8 > 512) ? 4096 / L : col_tx<T, L>();
-    constexpr int cap = OP == ZOP_SCALAR3 ? ZS3_THREADS : (OP == ZOP_VECTOR ? ZS2_THREADS : 1 << 30);
+    constexpr int cap = OP == ZOP_SCALAR3 ? 256 : (OP == ZOP_VECTOR ? 512 : 1 << 30);
     return (tx * L / 8 > cap && cap * 8 / L >= 1) ? cap * 8 / L : tx;
 }
 
@@ -992,36 +993,29 @@ template <typename T> static const cx<T> *twiddles_of(gev_ctx *c)
     else return c->tw32;
 }
 
-// forward x and y passes (r2c without the z pass) / inverse y and x passes
-template <typename T, int N> static void fwd_xy(gev_ctx *c, const T *in, cx<T> *out)
-{
-    launch_r2c<T, N>(in, out, c->P, (int64_t)N * N, twiddles_of<T>(c), c->stream);
-    launch_col<T, N>(out, c->P, 1, -1, twiddles_of<T>(c), c->stream);
-}
-template <typename T, int N> static void inv_yx(gev_ctx *c, cx<T> *in, T *out)
-{
-    launch_col<T, N>(in, c->P, 1, +1, twiddles_of<T>(c), c->stream);
-    launch_c2r<T, N>(in, out, c->P, (int64_t)N * N, twiddles_of<T>(c), c->stream);
-}
-
 template <typename T, int N>
 static void zsolve_chain(gev_ctx *c, int op, const T *rin, int nin, cx<T> *ftin, cx<T> *ftout, T *rout, int nout,
                          const ZParams &zp)
 {
-    if (op == ZOP_SCALAR) {
+    const cx<T> *tw = twiddles_of<T>(c);
+    if (op == ZOP_SCALAR && !plane_size(N)) {
         // x passes, then the y pass that forms the three groups of projectFTscalar
-        for (int i = 0; i < nin; i++)
-            launch_r2c<T, N>(rin + i * c->M, ftin + i * c->NK, c->P, (int64_t)N * N, twiddles_of<T>(c), c->stream);
-        launch_col_comb<T, N>(ftin, c->P, c->NK, twiddles_of<T>(c), zp, c->stream);
-        launch_zsolve<T, N, ZOP_SCALAR3>(ftin, ftout, c->P, c->NK, twiddles_of<T>(c), zp, c->stream);
+        if constexpr (!plane_size(N)) {
+            for (int i = 0; i < nin; i++)
+                launch_r2c<T, N>(rin + i * c->M, ftin + i * c->NK, c->P, (int64_t)N * N, tw, c->stream);
+            launch_col_comb<T, N>(ftin, c->P, c->NK, tw, zp, c->stream);
+            launch_zsolve<T, N, ZOP_SCALAR3>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
+        }
     } else {
-        for (int i = 0; i < nin; i++) fwd_xy<T, N>(c, rin + i * c->M, ftin + i * c->NK);
+        fwd_xy<T, N>(c, rin, ftin, nin, tw);
         if (op == ZOP_POISSON)
-            launch_zsolve<T, N, ZOP_POISSON>(ftin, ftout, c->P, c->NK, twiddles_of<T>(c), zp, c->stream);
-        else
-            launch_zsolve<T, N, ZOP_VECTOR>(ftin, ftout, c->P, c->NK, twiddles_of<T>(c), zp, c->stream);
+            launch_zsolve<T, N, ZOP_POISSON>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
+        else if (op == ZOP_VECTOR)
+            launch_zsolve<T, N, ZOP_VECTOR>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
+        else if constexpr (plane_size(N))
+            launch_zsolve<T, N, ZOP_SCALAR>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
     }
-    for (int j = 0; j < nout; j++) inv_yx<T, N>(c, ftout + j * c->NK, rout + j * c->M);
+    inv_yx<T, N>(c, ftout, rout, nout, tw);
 }
 
 template <typename T>
@@ -1029,18 +1023,16 @@ static int zsolve_dispatch(gev_ctx *c, int op, const T *rin, int nin, cx<T> *fti
                            const ZParams &zp)
 {
     switch (c->N) {
-    case 64: zsolve_chain<T, 64>(c, op, rin, nin, ftin, ftout, rout, nout, zp); break;
-    case 128: zsolve_chain<T, 128>(c, op, rin, nin, ftin, ftout, rout, nout, zp); break;
-    case 256: zsolve_chain<T, 256>(c, op, rin, nin, ftin, ftout, rout, nout, zp); break;
-    case 512: zsolve_chain<T, 512>(c, op, rin, nin, ftin, ftout, rout, nout, zp); break;
-    case 1024: zsolve_chain<T, 1024>(c, op, rin, nin, ftin, ftout, rout, nout, zp); break;
-    default: gev_set_error("fused z-pass solve needs 64 <= N <= 1024"); return GEV_ERR_ARG;
+#define X(n) case n: zsolve_chain<T, n>(c, op, rin, nin, ftin, ftout, rout, nout, zp); break;
+        GEV_FOR_FUSED_N(X)
+#undef X
+    default: gev_set_error("fused z-pass solve needs 16 <= N <= 1024"); return GEV_ERR_ARG;
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
 }
 
-bool zsolve_supported(const gev_ctx *c) { return c->N >= 64 && c->N <= 1024; }
+bool zsolve_supported(const gev_ctx *c) { return c->N >= 16 && c->N <= 1024; }
 
 // pot = c2r(poisson(r2c(src))) with the k=0 mode optionally replaced first
 template <typename T>
@@ -1048,42 +1040,73 @@ int solve_poisson_fused_impl(gev_ctx *c, const T *src, T *pot, cx<T> *work, doub
                              double k0re)
 {
     ZParams zp{c->gk2, c->kshift, coeff / -((double)c->N * (double)c->N * (double)c->N), modif, k0re, 0.0, k0set,
-               nullptr};
+               nullptr, 0, nullptr};
     return zsolve_dispatch<T>(c, ZOP_POISSON, src, 1, work, work, pot, 1, zp);
 }
 
+// A source written back over its input as it is formed (meshes below 128,
+// where gev_solve_poisson_T00 and gev_solve_chi_Tij leave the source terms in
+// place): each pair is read and written by the one thread that forms it.
+template <typename T, int N, class S> struct SrcPut : S {
+    T *dst;
+    __device__ __forceinline__ SrcPut(const S &s, T *d) : S(s), dst(d) {}
+    __device__ __forceinline__ cx<T> operator()(int64_t L, int n)
+    {
+        const cx<T> v = S::operator()(L, n);
+        reinterpret_cast<cx<T> *>(dst)[L * (N / 2) + n] = v;
+        return v;
+    }
+};
+
+template <typename T, int N> struct CompT00 {
+    SrcT00<T, N> s;
+    T *put;  // the source, written back for N < 128
+    template <class F> __device__ __forceinline__ void with(int, F f) const
+    {
+        if constexpr (N < 128) f(SrcPut<T, N, SrcT00<T, N>>(s, put));
+        else f(s);
+    }
+};
+
 // pot = c2r(poisson(r2c(prepareFTsource_T00(phi, chi, src)))) with the source
 // formed inside the x pass; its workgroup sums go to ctx->red + 64 and are
-// reduced to ctx->red[0] (source) and ctx->red[1] (result) before the z pass,
-// which takes the k=0 mode from ctx->red[1] when zp.k0set
+// reduced inside the z pass to ctx->red[0] (source) and ctx->red[1] (result),
+// which is the k=0 mode when zp.k0set
 template <typename T, int N>
-static void poisson_T00_chain(gev_ctx *c, const SrcT00<T, N> &src, T *pot, cx<T> *work, const ZParams &zp)
+static void poisson_T00_chain(gev_ctx *c, const SrcT00<T, N> &src, T *put, T *pot, cx<T> *work, ZParams zp)
 {
-    constexpr int NL = xlines<T, N>();
-    const int64_t nl = (int64_t)N * N, nb = (nl + NL - 1) / NL;
     const cx<T> *tw = twiddles_of<T>(c);
-    launch_r2c_src<T, N>(src, work, c->P, nl, tw, c->stream, c->red + 64);
-    launch_col<T, N>(work, c->P, 1, -1, tw, c->stream);
-    reduce_partials(c, c->red + 64, (int)nb, 2, c->red);
+    zp.parts = c->red + 64;
+    zp.sums = c->red;
+    if constexpr (plane_size(N)) {
+        zp.nparts = N / plane_np<N>();
+        launch_fwd_plane<T, N>(c, CompT00<T, N>{src, put}, work, 1, tw, c->red + 64);
+    } else {
+        constexpr int NL = xlines<T, N>();
+        const int64_t nl = (int64_t)N * N;
+        zp.nparts = (int)((nl + NL - 1) / NL);
+        launch_r2c_src<T, N>(src, work, c->P, nl, tw, c->stream, c->red + 64);
+        launch_col<T, N>(work, c->P, 1, -1, tw, c->stream);
+    }
     launch_zsolve<T, N, ZOP_POISSON>(work, work, c->P, c->NK, tw, zp, c->stream);
-    inv_yx<T, N>(c, work, pot);
+    inv_yx<T, N>(c, work, pot, 1, tw);
 }
 
 template <typename T>
-int solve_poisson_T00_fused_impl(gev_ctx *c, const T *phi, const T *chi, const T *src, double bg, double c1,
-                                 double c2, double c3, T *pot, cx<T> *work, double coeff, double modif, int k0set)
+int solve_poisson_T00_fused_impl(gev_ctx *c, const T *phi, const T *chi, T *src, double bg, double c1, double c2,
+                                 double c3, T *pot, cx<T> *work, double coeff, double modif, int k0set)
 {
     ZParams zp{c->gk2, c->kshift, coeff / -((double)c->N * (double)c->N * (double)c->N), modif, 0.0, 0.0, k0set,
-               k0set ? c->red + 1 : nullptr};
+               nullptr, 0, nullptr};
     switch (c->N) {
 #define X(n)                                                                                                     \
     case n:                                                                                                      \
-        poisson_T00_chain<T, n>(c, SrcT00<T, n>{phi, chi, src, (T)bg, (T)c1, (T)c2, (T)c3, {0.0, 0.0}}, pot, work, \
-                                zp);                                                                             \
+        poisson_T00_chain<T, n>(c, SrcT00<T, n>{phi, chi, src, (T)bg, (T)c1, (T)c2, (T)c3, {0.0, 0.0}}, src, pot, \
+                                work, zp);                                                                       \
         break;
-        X(128) X(256) X(512) X(1024)
+        GEV_FOR_FUSED_N(X)
 #undef X
-    default: gev_set_error("prepareFTsource T00 inside the Poisson solve needs 128 <= N <= 1024"); return GEV_ERR_ARG;
+    default: gev_set_error("prepareFTsource T00 inside the Poisson solve needs 16 <= N <= 1024"); return GEV_ERR_ARG;
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
@@ -1092,35 +1115,63 @@ int solve_poisson_T00_fused_impl(gev_ctx *c, const T *phi, const T *chi, const T
 // chi = c2r(projectFTscalar(r2c(Sij)))
 template <typename T> int solve_chi_fused_impl(gev_ctx *c, const T *Sij, T *chi, cx<T> *SijFT, cx<T> *chiFT)
 {
-    ZParams zp{c->gk2, c->kshift, 0.0, 0.0, 0.0, 0.0, 0, nullptr};
+    ZParams zp{c->gk2, c->kshift, 0.0, 0.0, 0.0, 0.0, 0, nullptr, 0, nullptr};
     return zsolve_dispatch<T>(c, ZOP_SCALAR, Sij, 6, SijFT, chiFT, chi, 1, zp);
 }
 
+template <typename T, int N> struct CompSij {
+    const T *phi;
+    T *Tij;
+    int64_t M;
+    T coeff;
+    template <class F> __device__ __forceinline__ void with(int c, F f) const
+    {
+        auto one = [&](auto cc) {
+            constexpr int C = decltype(cc)::value;
+            const SrcSij<T, N, C> s{phi, Tij + C * M, coeff};
+            if constexpr (N < 128) f(SrcPut<T, N, SrcSij<T, N, C>>(s, Tij + C * M));
+            else f(s);
+        };
+        switch (c) {
+        case 0: one(std::integral_constant<int, 0>{}); break;
+        case 1: one(std::integral_constant<int, 1>{}); break;
+        case 2: one(std::integral_constant<int, 2>{}); break;
+        case 3: one(std::integral_constant<int, 3>{}); break;
+        case 4: one(std::integral_constant<int, 4>{}); break;
+        default: one(std::integral_constant<int, 5>{}); break;
+        }
+    }
+};
+
 // chi from Tij: the x passes compute Sij = prepareFTsource(phi, Tij, coeff)
-// on the fly (N >= 128; the caller runs the unfused sequence below that)
+// on the fly (and write it over Tij below N = 128)
 template <typename T, int N>
-static void chi_from_Tij_chain(gev_ctx *c, const T *phi, const T *Tij, T coeff, cx<T> *SijFT, cx<T> *chiFT, T *chi)
+static void chi_from_Tij_chain(gev_ctx *c, const T *phi, T *Tij, T coeff, cx<T> *SijFT, cx<T> *chiFT, T *chi)
 {
     const int64_t nl = (int64_t)N * N;
     const cx<T> *tw = twiddles_of<T>(c);
-    launch_r2c_multi<T, N, 6>(SrcSij6<T, N>{phi, Tij, c->M, coeff}, SijFT, c->P, c->NK, nl, tw, c->stream);
-    ZParams zp{c->gk2, c->kshift, 0.0, 0.0, 0.0, 0.0, 0, nullptr};
-    launch_col_comb<T, N>(SijFT, c->P, c->NK, tw, zp, c->stream);
-    launch_zsolve<T, N, ZOP_SCALAR3>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
-    inv_yx<T, N>(c, chiFT, chi);
+    ZParams zp{c->gk2, c->kshift, 0.0, 0.0, 0.0, 0.0, 0, nullptr, 0, nullptr};
+    if constexpr (plane_size(N)) {
+        launch_fwd_plane<T, N>(c, CompSij<T, N>{phi, Tij, c->M, coeff}, SijFT, 6, tw);
+        launch_zsolve<T, N, ZOP_SCALAR>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
+    } else {
+        launch_r2c_multi<T, N, 6>(SrcSij6<T, N>{phi, Tij, c->M, coeff}, SijFT, c->P, c->NK, nl, tw, c->stream);
+        launch_col_comb<T, N>(SijFT, c->P, c->NK, tw, zp, c->stream);
+        launch_zsolve<T, N, ZOP_SCALAR3>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
+    }
+    inv_yx<T, N>(c, chiFT, chi, 1, tw);
 }
 
-bool chi_from_Tij_supported(const gev_ctx *c) { return c->N >= 128 && c->N <= 1024; }
+bool fused_sources_supported(const gev_ctx *c) { return c->N >= 16 && c->N <= 1024; }
 
 template <typename T>
-int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, const T *Tij, double coeff, T *chi, cx<T> *SijFT, cx<T> *chiFT)
+int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, T *Tij, double coeff, T *chi, cx<T> *SijFT, cx<T> *chiFT)
 {
     switch (c->N) {
-    case 128: chi_from_Tij_chain<T, 128>(c, phi, Tij, (T)coeff, SijFT, chiFT, chi); break;
-    case 256: chi_from_Tij_chain<T, 256>(c, phi, Tij, (T)coeff, SijFT, chiFT, chi); break;
-    case 512: chi_from_Tij_chain<T, 512>(c, phi, Tij, (T)coeff, SijFT, chiFT, chi); break;
-    case 1024: chi_from_Tij_chain<T, 1024>(c, phi, Tij, (T)coeff, SijFT, chiFT, chi); break;
-    default: gev_set_error("chi from Tij needs 128 <= N <= 1024"); return GEV_ERR_ARG;
+#define X(n) case n: chi_from_Tij_chain<T, n>(c, phi, Tij, (T)coeff, SijFT, chiFT, chi); break;
+        GEV_FOR_FUSED_N(X)
+#undef X
+    default: gev_set_error("chi from Tij needs 16 <= N <= 1024"); return GEV_ERR_ARG;
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
@@ -1129,25 +1180,40 @@ int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, const T *Tij, double coef
 // Bi = c2r(projectFTvector(r2c(Bi))), in place on Bi
 template <typename T> int solve_vector_fused_impl(gev_ctx *c, T *Bi, cx<T> *BiFT, double coeff, double modif)
 {
-    ZParams zp{c->gk2, c->kshift, coeff, modif, 0.0, 0.0, 0, nullptr};
+    ZParams zp{c->gk2, c->kshift, coeff, modif, 0.0, 0.0, 0, nullptr, 0, nullptr};
     return zsolve_dispatch<T>(c, ZOP_VECTOR, Bi, 3, BiFT, BiFT, Bi, 3, zp);
 }
+
+template <typename T, int N> struct CompLink {
+    const T *phi, *L;
+    int64_t M;
+    template <class F> __device__ __forceinline__ void with(int c, F f) const
+    {
+        if (c == 0) f(SrcT0iLink<T, N, 0>{phi, L});
+        else if (c == 1) f(SrcT0iLink<T, N, 1>{phi, L + M});
+        else f(SrcT0iLink<T, N, 2>{phi, L + 2 * M});
+    }
+};
 
 // the same from T0i link sums: the x passes apply the link factor with phi
 template <typename T, int N>
 static void vector_from_links_chain(gev_ctx *c, T *Bi, const T *phi, cx<T> *BiFT, const ZParams &zp)
 {
-    const int64_t nl = (int64_t)N * N, M = c->M;
     const cx<T> *tw = twiddles_of<T>(c);
-    auto xy = [&](const auto &src, int i) {
-        launch_r2c_src<T, N>(src, BiFT + i * c->NK, c->P, nl, tw, c->stream);
-        launch_col<T, N>(BiFT + i * c->NK, c->P, 1, -1, tw, c->stream);
-    };
-    xy(SrcT0iLink<T, N, 0>{phi, Bi}, 0);
-    xy(SrcT0iLink<T, N, 1>{phi, Bi + M}, 1);
-    xy(SrcT0iLink<T, N, 2>{phi, Bi + 2 * M}, 2);
+    if constexpr (plane_size(N)) {
+        launch_fwd_plane<T, N>(c, CompLink<T, N>{phi, Bi, c->M}, BiFT, 3, tw);
+    } else {
+        const int64_t nl = (int64_t)N * N, M = c->M;
+        auto xy = [&](const auto &src, int i) {
+            launch_r2c_src<T, N>(src, BiFT + i * c->NK, c->P, nl, tw, c->stream);
+            launch_col<T, N>(BiFT + i * c->NK, c->P, 1, -1, tw, c->stream);
+        };
+        xy(SrcT0iLink<T, N, 0>{phi, Bi}, 0);
+        xy(SrcT0iLink<T, N, 1>{phi, Bi + M}, 1);
+        xy(SrcT0iLink<T, N, 2>{phi, Bi + 2 * M}, 2);
+    }
     launch_zsolve<T, N, ZOP_VECTOR>(BiFT, BiFT, c->P, c->NK, tw, zp, c->stream);
-    for (int j = 0; j < 3; j++) inv_yx<T, N>(c, BiFT + j * c->NK, Bi + j * M);
+    inv_yx<T, N>(c, BiFT, Bi, 3, tw);
 }
 
 // the link factor alone, in place (meshes below the fused chain's range)
@@ -1174,26 +1240,25 @@ template <typename T> int t0i_link_factor_impl(gev_ctx *c, T *Bi, const T *phi)
 template <typename T>
 int solve_vector_links_fused_impl(gev_ctx *c, T *Bi, const T *phi, cx<T> *BiFT, double coeff, double modif)
 {
-    ZParams zp{c->gk2, c->kshift, coeff, modif, 0.0, 0.0, 0, nullptr};
+    ZParams zp{c->gk2, c->kshift, coeff, modif, 0.0, 0.0, 0, nullptr, 0, nullptr};
     switch (c->N) {
-    case 128: vector_from_links_chain<T, 128>(c, Bi, phi, BiFT, zp); break;
-    case 256: vector_from_links_chain<T, 256>(c, Bi, phi, BiFT, zp); break;
-    case 512: vector_from_links_chain<T, 512>(c, Bi, phi, BiFT, zp); break;
-    case 1024: vector_from_links_chain<T, 1024>(c, Bi, phi, BiFT, zp); break;
-    default: gev_set_error("B from T0i links needs 128 <= N <= 1024"); return GEV_ERR_ARG;
+#define X(n) case n: vector_from_links_chain<T, n>(c, Bi, phi, BiFT, zp); break;
+        GEV_FOR_FUSED_N(X)
+#undef X
+    default: gev_set_error("B from T0i links needs 16 <= N <= 1024"); return GEV_ERR_ARG;
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
 }
 
 #define INSTZ(T)                                                                                       \
-    template int solve_chi_Tij_fused_impl<T>(gev_ctx *, const T *, const T *, double, T *, cx<T> *, cx<T> *); \
+    template int solve_chi_Tij_fused_impl<T>(gev_ctx *, const T *, T *, double, T *, cx<T> *, cx<T> *);  \
     template int solve_poisson_fused_impl<T>(gev_ctx *, const T *, T *, cx<T> *, double, double, int, double); \
     template int solve_chi_fused_impl<T>(gev_ctx *, const T *, T *, cx<T> *, cx<T> *);                  \
     template int solve_vector_fused_impl<T>(gev_ctx *, T *, cx<T> *, double, double);                    \
     template int solve_vector_links_fused_impl<T>(gev_ctx *, T *, const T *, cx<T> *, double, double);    \
     template int t0i_link_factor_impl<T>(gev_ctx *, T *, const T *);                                      \
-    template int solve_poisson_T00_fused_impl<T>(gev_ctx *, const T *, const T *, const T *, double, double, double, \
+    template int solve_poisson_T00_fused_impl<T>(gev_ctx *, const T *, const T *, T *, double, double, double, \
                                                  double, T *, cx<T> *, double, double, int);
 INSTZ(double)
 INSTZ(float)

@@ -1,6 +1,6 @@
 // gev_fft_engine.hpp -- register-staged Stockham FFT for one workgroup.
 //
-// A workgroup transforms NL lines of length L (power of two, L >= 64) with
+// A workgroup transforms NL lines of length L (power of two, L >= 8) with
 // NL*L/8 threads; every thread owns one radix-8 butterfly slot per stage
 // (two radix-4 or four radix-2 butterflies in a trailing stage).  The first
 // stage reads its operands straight from a caller functor (global memory or
@@ -53,23 +53,30 @@ template <typename T, int R> __device__ __forceinline__ void dftR(cx<T> *v, int 
     else dft2(v);
 }
 
+// where element `pos` of line `line` sits in the exchange buffer
+template <int LDL> struct LineAddr {
+    __device__ __forceinline__ int operator()(int line, int pos) const { return line * LDL + pos; }
+};
+
 // LF (line-fast): consecutive threads walk lines first (coalesced when lines
 // are adjacent columns in memory); otherwise they walk along a line.
 // The store functor is called as st(line, pos, value, slot) with slot in
 // [0, 8) a compile-time constant per call site: the thread's slot-th output,
 // always at the same (line, pos) for a given thread and L, NL, LF.
 // twl[m * TWS] = exp(-2 pi i m / L).  ST_LDS: the store functor writes the
-// same LDS buffer, so the last stage waits for all reads first.
-template <typename T, int L, int NL, bool LF, int TWS, bool ST_LDS, int NS, class LD, class ST>
-__device__ __forceinline__ void reg_fft(cx<T> *lds, const cx<T> *twl, int dir, LD &ld, ST &st)
+// same LDS buffer, so the last stage waits for all reads first.  hook() runs
+// once the first stage's operands are requested; what it writes to LDS is
+// visible from the second stage on.
+template <typename T, int L, int NL, bool LF, int TWS, bool ST_LDS, int NS, class AD, class LD, class ST, class HK>
+__device__ __forceinline__ void reg_fft_at(cx<T> *lds, const cx<T> *twl, int dir, const AD &ad, LD &ld, ST &st,
+                                           const HK &hook)
 {
     constexpr int REM = L / NS;
     constexpr int R = REM >= 8 ? 8 : REM;
     constexpr int BPT = 8 / R;
     constexpr int NB = L / R;
     constexpr bool FIRST = (NS == 1), LAST = (NS * R == L);
-    constexpr int LDL = L + 1;
-    static_assert(L >= 64, "reg_fft needs L >= 64");
+    static_assert(L >= 8, "eight values per thread");
     const int t = threadIdx.x;
     const int line = LF ? t % NL : t / (L / 8);
     const int jt = LF ? t / NL : t % (L / 8);
@@ -80,7 +87,11 @@ __device__ __forceinline__ void reg_fft(cx<T> *lds, const cx<T> *twl, int dir, L
 #pragma unroll
         for (int r = 0; r < R; r++) {
             if constexpr (FIRST) v[u][r] = ld(line, j + r * NB);
-            else v[u][r] = lds[line * LDL + j + r * NB];
+            else v[u][r] = lds[ad(line, j + r * NB)];
+        }
+        if constexpr (FIRST) {
+            static_assert(BPT == 1, "the first stage is radix 8");
+            hook();
         }
         if constexpr (NS > 1) {
             const int k = j % NS;
@@ -107,11 +118,48 @@ __device__ __forceinline__ void reg_fft(cx<T> *lds, const cx<T> *twl, int dir, L
         for (int u = 0; u < BPT; u++) {
             const int j = jt * BPT + u;
 #pragma unroll
-            for (int r = 0; r < R; r++) lds[line * LDL + (j / NS) * NS * R + (j % NS) + r * NS] = v[u][r];
+            for (int r = 0; r < R; r++) lds[ad(line, (j / NS) * NS * R + (j % NS) + r * NS)] = v[u][r];
         }
         __syncthreads();
-        reg_fft<T, L, NL, LF, TWS, ST_LDS, NS * R, LD, ST>(lds, twl, dir, ld, st);
+        reg_fft_at<T, L, NL, LF, TWS, ST_LDS, NS * R, AD, LD, ST, HK>(lds, twl, dir, ad, ld, st, hook);
     }
 }
+
+struct NoHook {
+    __device__ __forceinline__ void operator()() const {}
+};
+
+// lines of pitch L + 1 (consecutive lines start in different LDS banks)
+template <typename T, int L, int NL, bool LF, int TWS, bool ST_LDS, int NS, class LD, class ST, class HK = NoHook>
+__device__ __forceinline__ void reg_fft(cx<T> *lds, const cx<T> *twl, int dir, LD &ld, ST &st, const HK &hook = HK{})
+{
+    reg_fft_at<T, L, NL, LF, TWS, ST_LDS, NS>(lds, twl, dir, LineAddr<L + 1>{}, ld, st, hook);
+}
+
+// The twiddle table on its way to LDS: requested from memory when this is
+// made, stored by operator() -- as a transform's hook, after its operands are
+// requested, so the table's round trip and theirs overlap instead of a
+// barrier between them.
+template <typename T, int L, int NT> struct TwiddleLoad {
+    static constexpr int K = (L + NT - 1) / NT;
+    cx<T> v[K];
+    cx<T> *twl;
+    __device__ __forceinline__ TwiddleLoad(cx<T> *twl_, const cx<T> *__restrict__ tw) : twl(twl_)
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int m = threadIdx.x + k * NT;
+            v[k] = (L % NT == 0 || m < L) ? tw[m] : mk((T)0, (T)0);
+        }
+    }
+    __device__ __forceinline__ void operator()() const
+    {
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            const int m = threadIdx.x + k * NT;
+            if (L % NT == 0 || m < L) twl[m] = v[k];
+        }
+    }
+};
 
 }  // namespace gev

@@ -21,25 +21,28 @@ int ic_displacement_ft_impl(gev_ctx *ctx, uint32_t seed, int ksphere, double coe
 template <typename T> int set_k0_impl(gev_ctx *ctx, cx<T> *ft, double re, double im);
 
 // r2c -> k-space operator -> c2r with the operator applied inside the z pass
-// (64 <= N <= 1024); the FT arguments are work space of the usual layout
+// (16 <= N <= 1024); the FT arguments are work space of the usual layout
 bool zsolve_supported(const gev_ctx *c);
-bool chi_from_Tij_supported(const gev_ctx *c);
+// the sources formed inside the solves' x passes (16 <= N <= 1024)
+bool fused_sources_supported(const gev_ctx *c);
 template <typename T>
 int solve_poisson_fused_impl(gev_ctx *c, const T *src, T *pot, cx<T> *work, double coeff, double modif, int k0set,
                              double k0re);
 template <typename T> int solve_chi_fused_impl(gev_ctx *c, const T *Sij, T *chi, cx<T> *SijFT, cx<T> *chiFT);
+// below N = 128 Tij is overwritten with Sij
 template <typename T>
-int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, const T *Tij, double coeff, T *chi, cx<T> *SijFT, cx<T> *chiFT);
+int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, T *Tij, double coeff, T *chi, cx<T> *SijFT, cx<T> *chiFT);
 template <typename T> int solve_vector_fused_impl(gev_ctx *c, T *Bi, cx<T> *BiFT, double coeff, double modif);
 // Bi holds T0i link sums (no 1 + phi_a + phi_b factor) on entry, B on return
-// (128 <= N <= 1024, as chi_from_Tij_supported)
+// (16 <= N <= 1024)
 template <typename T>
 int solve_vector_links_fused_impl(gev_ctx *c, T *Bi, const T *phi, cx<T> *BiFT, double coeff, double modif);
-// prepareFTsource T00 form formed inside the Poisson solve's x pass (128 <= N
-// <= 1024); ctx->red[0] / ctx->red[1] receive the FP64 sums of the source and
-// of the result, and the k=0 mode is taken from ctx->red[1] when k0set
+// prepareFTsource T00 form formed inside the Poisson solve's x pass (16 <= N
+// <= 1024; below 128 it is also written over src); ctx->red[0] / ctx->red[1]
+// receive the FP64 sums of the source and of the result, and the k=0 mode is
+// taken from ctx->red[1] when k0set
 template <typename T>
-int solve_poisson_T00_fused_impl(gev_ctx *c, const T *phi, const T *chi, const T *src, double bg, double c1,
+int solve_poisson_T00_fused_impl(gev_ctx *c, const T *phi, const T *chi, T *src, double bg, double c1,
                                  double c2, double c3, T *pot, cx<T> *work, double coeff, double modif, int k0set);
 // Bi[c] *= 1 + phi(x) + phi(x + e_c), in place
 template <typename T> int t0i_link_factor_impl(gev_ctx *c, T *Bi, const T *phi);

@@ -134,7 +134,7 @@ int gev_set_k0(gev_ctx *ctx, void *ft, double re, double im);
 
 /* ---- fused real-space solves.  No single reference function: each is one
  *      main.cu call sequence with the k-space operator applied inside the z
- *      pass of the transforms (64 <= N <= 1024; smaller N runs the sequence
+ *      pass of the transforms (16 <= N <= 1024; smaller N runs the sequence
  *      unfused).  Work buffers are Fourier fields of the usual layout; their
  *      content is undefined afterwards. */
 /* plan_source FFT_FORWARD, [k=0 := k0_re], solveModifiedPoissonFT, plan_phi
@@ -144,17 +144,17 @@ int gev_solve_poisson(gev_ctx *ctx, const void *src, void *pot, void *workFT, do
 /* plan_Sij FFT_FORWARD, projectFTscalar (add = 0), plan_chi FFT_BACKWARD (main.cu:829-895) */
 int gev_solve_chi(gev_ctx *ctx, const void *Sij, void *chi, void *SijFT, void *chiFT);
 /* prepareFTsource<Cplx>(phi, Sij, Sij, coeff) (gevolution.hpp:64-119,
- * main.cu:822-828) followed by gev_solve_chi: for 128 <= N <= 1024 the x
- * passes read Tij and phi and form Sij on the fly, so Sij is never stored;
- * Tij is left unchanged there and holds Sij on return for smaller N. */
+ * main.cu:822-828) followed by gev_solve_chi: the x passes read Tij and phi
+ * and form Sij on the fly (16 <= N <= 1024).  For N >= 128 Tij is left
+ * unchanged; it holds Sij on return for smaller N. */
 int gev_solve_chi_Tij(gev_ctx *ctx, const void *phi, void *Tij, double coeff, void *chi, void *SijFT, void *chiFT);
 /* plan_Bi FFT_FORWARD, projectFTvector, plan_Bi FFT_BACKWARD (main.cu:918-948), Bi in place */
 int gev_solve_vector(gev_ctx *ctx, void *Bi, void *BiFT, double coeff, double modif);
 /* prepareFTsource, T00 form (gevolution.hpp:160-183; main.cu:725), and
  * solveModifiedPoissonFT with its transforms (main.cu:742-794) in one chain,
- * pot = phi allowed: for 128 <= N <= 1024 the source is formed inside the
- * forward x pass and never stored, and source is only read; below that the
- * source pass runs in place over source first.  k0set: the k=0 mode of the
+ * pot = phi allowed: for 16 <= N <= 1024 the source is formed inside the
+ * forward x pass.  For N >= 128 it is never stored and source is only read;
+ * below that source holds the source terms on return.  k0set: the k=0 mode of the
  * transformed source becomes the FP64 sum of the source terms (as
  * gev_solve_poisson with k0re = sums[1]).  sums (may be NULL): the FP64 sums
  * of source and of the source terms, as gev_prepare_source_T00 returns them;
@@ -167,7 +167,7 @@ int gev_solve_poisson_T00(gev_ctx *ctx, const void *phi, const void *chi, void *
 int gev_ctx_sums(gev_ctx *ctx, double sums[2]);
 /* gev_solve_vector of T0i given as link sums (gev_project_T00_Tij_T0i_links):
  * Bi[c](x) *= 1 + phi(x) + phi(x + e_c), then the solve; for
- * 128 <= N <= 1024 the factor is applied inside the forward x passes. */
+ * 16 <= N <= 1024 the factor is applied inside the forward x passes. */
 int gev_solve_vector_T0i_links(gev_ctx *ctx, void *Bi, const void *phi, void *BiFT, double coeff, double modif);
 
 /* ---- particle updates (perfParticles::updateVel / moveParticles with the
