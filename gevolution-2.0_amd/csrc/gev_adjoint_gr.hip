@@ -28,18 +28,6 @@
 #include "gev_kops.hpp"
 #include "gev_pcommon.hpp"
 
-// FP32 tiles of the reverse kick/drift and deposit: 1 the wide ones
-// (16 x 8 x 8), 0 the 8 x 8 x 4 ones (more workgroups per CU, more halo)
-#ifndef ADJ_KD_WIDE
-#define ADJ_KD_WIDE 1
-#endif
-#ifndef ADJ_DEP_WIDE
-#define ADJ_DEP_WIDE 1
-#endif
-#ifndef ADJ_CHUNK_X4
-#define ADJ_CHUNK_X4 1  // four times the mean particles per tile cell from which the reverse kick/drift walks per-lane chunks
-#endif
-
 namespace gev {
 
 template <typename T> __device__ __forceinline__ void gadd(T *p, double v) { atomicAdd(p, (T)v); }
@@ -80,8 +68,8 @@ template <typename R> struct CubeAt {
 // B_l along l times the trilinear weights across) and the three mixed
 // differences M[l] = d^2 B_l / dr_a dr_b over the cube, a, b the other two
 // axes (dP[0][1]/dr_2 = dP[2][1]/dr_0 = M[1], and so on)
-template <typename R, class FA>
-__device__ __forceinline__ void pgrad_matrix(const FA &B0, const FA &B1, const FA &B2, const R r[3], R P[3][3],
+template <typename R, class F0, class F1, class F2>
+__device__ __forceinline__ void pgrad_matrix(const F0 &B0, const F1 &B1, const F2 &B2, const R r[3], R P[3][3],
                                              R dPd[3][3], R M[3])
 {
     const R o = (R)1, s0 = o - r[0], s1 = o - r[1], s2 = o - r[2];
@@ -120,15 +108,17 @@ __device__ __forceinline__ void pgrad_matrix(const FA &B0, const FA &B1, const F
     diag(2, [&](int t, int u, int v) { return B2(u, v, t); });
 }
 
+// with the quotients every particle needs, formed once on the host: K = dtau_k
+// N, 1 / bc_k, 1 / bc_d, K / bc_k and dtau_d / bc_d
 struct AdjKD {
     int nf_k, nf_d;
-    double a_k, a_d, dtau_k, dtau_d, bc_k, bc_d;
+    double a_k, a_d, dtau_k, dtau_d, bc_k, bc_d, K, ibk, ibd, K_bk, d_bd;
 };
 
 // Reverse of the fused kick + drift of one particle (state before the kick),
 // at cell offsets r and momenta q, with the adjoints LX, LQ after the drift:
 // nx, nq the adjoints before the kick; the fields' adjoints go to
-// sc(f, dx, dy, dz, value) with f = 0 phi, 1 chi, 2..4 B_x..B_z and the
+// sc(F, dx, dy, dz, value) with F the accessor of the field and the
 // site's offset from the particle's cell.  Fields are read through the
 // accessors Fp, Fc, FB0..FB2 (offsets from the particle's cell).
 //
@@ -143,9 +133,9 @@ struct AdjKD {
 // off-diagonal (d(mu.b)/dr_j = sum_{l != j} mu_l P[j][l]).  Its reverse is
 // written out term by term: one pass over the stencil per particle in place
 // of six forward tangent directions.
-template <typename T, class FA, class SC>
-__device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], const T LX[3], const T LQ[3], const FA &Fp,
-                                                const FA &Fc, const FA &FB0, const FA &FB1, const FA &FB2, int N,
+template <typename T, class FP, class FC, class F0, class F1, class F2, class SC>
+__device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], const T LX[3], const T LQ[3], const FP &Fp,
+                                                const FC &Fc, const F0 &FB0, const F1 &FB1, const F2 &FB2, int N,
                                                 const AdjKD &s, T nx[3], T nq[3], SC &sc)
 {
     // in the container's precision (FP32 for the mixed form)
@@ -154,9 +144,10 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
     const R q[3] = {qt[0], qt[1], qt[2]};
     const R Nd = (R)N;
     const R o = (R)1;
-    const int nfm = s.nf_k > s.nf_d ? s.nf_k : s.nf_d;
+    const int nf_k = s.nf_k, nf_d = s.nf_d;
+    const int nfm = nf_k > nf_d ? nf_k : nf_d;
     // ---- the kick, keeping what its reverse needs
-    const R K = (R)(s.dtau_k * N);
+    const R K = (R)s.K;
     const R a2k = (R)(s.a_k * s.a_k);
     const R v2 = q[0] * q[0] + q[1] * q[1] + q[2] * q[2];
     const R e2 = v2 + a2k, ie2 = o / e2, e = sqrt(e2);
@@ -165,15 +156,15 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
     grad1<R>(Fp, r, gP);  // dPhi/dr
     grad2<R>(Fp, r, G2);
     if (nfm >= 2) grad1<R>(Fc, r, G1);
-    const R Chi = s.nf_d >= 2 ? cic<R>(Fc, r) : (R)0;
+    const R Chi = nf_d >= 2 ? cic<R>(Fc, r) : (R)0;
     R P[3][3] = {}, dPd[3][3] = {}, Mx[3] = {};
     if (nfm >= 3) pgrad_matrix<R>(FB0, FB1, FB2, r, P, dPd, Mx);
     const R p1 = Phi * ie2;
     const R Phibar = (R)4 * p1 * v2 + (o + a2k * p1) * (v2 + e2) * ie2;
     const R dPhibar = ((R)4 * v2 + a2k * (v2 + e2) * ie2) * ie2;  // dPhibar/dPhi
     const R dPbv = a2k * ie2 * ie2 * (((R)4 * Phi + o) - (R)2 * Phi * v2 * ie2);  // dPhibar/dv2 (e^2 = v2 + a_k^2)
-    const R k2 = s.nf_k >= 2 ? o : (R)0;
-    const R ibk = s.nf_k >= 3 ? (R)(1.0 / s.bc_k) : (R)0;
+    const R k2 = nf_k >= 2 ? o : (R)0;
+    const R ibk = nf_k >= 3 ? (R)s.ibk : (R)0;
     R qq[3];
 #pragma unroll
     for (int l = 0; l < 3; l++)
@@ -182,7 +173,7 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
     const R a2d = (R)(s.a_d * s.a_d);
     const R w2 = qq[0] * qq[0] + qq[1] * qq[1] + qq[2] * qq[2];
     const R f2 = w2 + a2d, ie = o / sqrt(f2), ie_2 = ie * ie, ie3 = ie * ie_2;
-    const R ph = s.nf_d >= 1 ? Phi : (R)0;
+    const R ph = nf_d >= 1 ? Phi : (R)0;
     const R dtd = (R)s.dtau_d;
     const R mu[3] = {dtd * LX[0], dtd * LX[1], dtd * LX[2]};
     const R mq = mu[0] * qq[0] + mu[1] * qq[1] + mu[2] * qq[2];
@@ -194,8 +185,8 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
     R lqt[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) lqt[j] = LQ[j] + mu[j] * fac + (R)2 * mq * dfac * qq[j];
-    const R ibd = s.nf_d >= 3 ? (R)(1.0 / s.bc_d) : (R)0;
-    const R cph = s.nf_d >= 1 ? mq * ie * t3 : (R)0, cch = s.nf_d >= 2 ? mq * ie : (R)0;
+    const R ibd = nf_d >= 3 ? (R)s.ibd : (R)0;
+    const R cph = nf_d >= 1 ? mq * ie * t3 : (R)0, cch = nf_d >= 2 ? mq * ie : (R)0;
     R ar[3];
     ar[0] = cph * gP[0] - cch * G1[0] + ibd * (mu[1] * P[0][1] + mu[2] * P[0][2]);
     ar[1] = cph * gP[1] - cch * G1[1] + ibd * (mu[0] * P[1][0] + mu[2] * P[1][2]);
@@ -223,7 +214,7 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
     R kr[3];
 #pragma unroll
     for (int j = 0; j < 3; j++) kr[j] = e * (lg2 * dPhibar * gP[j] + Phibar * dlg2[j]);
-    if (s.nf_k >= 2) {
+    if (nf_k >= 2) {
         // lambda.G1 = sum_l lambda_l dChi/dr_l: its r-gradient takes the mixed
         // second differences of chi over the cube
         const R s0 = o - r[0], s1 = o - r[1], s2 = o - r[2];
@@ -237,7 +228,7 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
         kr[1] -= e * (lqt[0] * H01 + lqt[2] * H12);
         kr[2] -= e * (lqt[0] * H02 + lqt[1] * H12);
     }
-    if (s.nf_k >= 3) {
+    if (nf_k >= 3) {
         // lambda . P q: the diagonal's own r-derivatives and the mixed ones
         const R l0 = lqt[0], l1 = lqt[1], l2 = lqt[2];
         kr[0] += ibk * (l0 * q[0] * dPd[0][0] + l1 * (q[1] * dPd[1][0] + q[2] * Mx[2]) +
@@ -261,13 +252,13 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
         for (int i = 0; i < 64; i++) st[i >> 4][(i >> 2) & 3][i & 3] = (R)0;
     };
     auto add = [&](int dx, int dy, int dz, R val) { st[dx + 1][dy + 1][dz + 1] += val; };
-    auto put = [&](int f, int dx, int dy, int dz) { sc(f, dx, dy, dz, st[dx + 1][dy + 1][dz + 1]); };
+    auto put = [&](const auto &F, int dx, int dy, int dz) { sc(F, dx, dy, dz, st[dx + 1][dy + 1][dz + 1]); };
     // phi: g = Phibar grad2(phi) - grad1(chi) + pgradB / (bcoeff e); q' = q - K e g
     {
         clear();
         const R lG2[3] = {-K * e * Phibar * lqt[0], -K * e * Phibar * lqt[1], -K * e * Phibar * lqt[2]};
         const R lPhi = -K * e * dPhibar * lg2;
-        const R lph = s.nf_d >= 1 ? dtd * qL * t3 * ie : (R)0;
+        const R lph = nf_d >= 1 ? dtd * qL * t3 * ie : (R)0;
 #pragma unroll
         for (int b = 0; b < 8; b++) {
             const int bx = (b >> 2) & 1, by = (b >> 1) & 1, bz = b & 1;
@@ -284,18 +275,18 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
 #pragma unroll
         for (int b = 0; b < 8; b++) {
             const int u = (b >> 2) & 1, v_ = (b >> 1) & 1, w_ = b & 1;
-            put(0, u, v_, w_);                              // the cube
+            put(Fp, u, v_, w_);                              // the cube
         }
 #pragma unroll
         for (int b = 0; b < 4; b++) {
             const int u = (b >> 1) & 1, v_ = b & 1;
-            put(0, -1, u, v_); put(0, 2, u, v_);            // x faces
-            put(0, u, -1, v_); put(0, u, 2, v_);            // y faces
-            put(0, u, v_, -1); put(0, u, v_, 2);            // z faces
+            put(Fp, -1, u, v_); put(Fp, 2, u, v_);            // x faces
+            put(Fp, u, -1, v_); put(Fp, u, 2, v_);            // y faces
+            put(Fp, u, v_, -1); put(Fp, u, v_, 2);            // z faces
         }
     }
     // chi: the kick's -grad1(chi) and the drift's -chi
-    if (s.nf_k >= 2 || s.nf_d >= 2) {
+    if (nf_k >= 2 || nf_d >= 2) {
         clear();
         const R lG1[3] = {K * e * lqt[0], K * e * lqt[1], K * e * lqt[2]};
         const R lch = (R)(-s.dtau_d * qL * ie);
@@ -303,23 +294,23 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
         for (int b = 0; b < 8; b++) {
             const int bx = (b >> 2) & 1, by = (b >> 1) & 1, bz = b & 1;
             R val = (R)0;
-            if (s.nf_k >= 2) {
+            if (nf_k >= 2) {
                 R gw[3];
                 cw_grad(b, r, gw);
                 val += gw[0] * lG1[0] + gw[1] * lG1[1] + gw[2] * lG1[2];
             }
-            if (s.nf_d >= 2) val += cw(b, r) * lch;
+            if (nf_d >= 2) val += cw(b, r) * lch;
             add(bx, by, bz, val);
         }
 #pragma unroll
-        for (int b = 0; b < 8; b++) put(1, (b >> 2) & 1, (b >> 1) & 1, b & 1);
+        for (int b = 0; b < 8; b++) put(Fc, (b >> 2) & 1, (b >> 1) & 1, b & 1);
     }
     // B: pgradB (gevolution.hpp:968-994) is linear in B, its transpose term by
     // term; the drift's staggered B interpolation (:1213-1226)
-    if (s.nf_k >= 3 || s.nf_d >= 3) {
-        const R c = s.nf_k >= 3 ? -K / s.bc_k : (R)0;
+    if (nf_k >= 3 || nf_d >= 3) {
+        const R c = nf_k >= 3 ? (R)-s.K_bk : (R)0;
         const R l0 = c * lqt[0], l1 = c * lqt[1], l2 = c * lqt[2];
-        const R cd = s.nf_d >= 3 ? (R)(s.dtau_d / s.bc_d) : (R)0;
+        const R cd = nf_d >= 3 ? (R)s.d_bd : (R)0;
         const R b0 = cd * LX[0], b1 = cd * LX[1], b2 = cd * LX[2];
         const R s0 = o - r[0], s1 = o - r[1], s2 = o - r[2];
         // B0: x stencil of pg[0], the y and z links of pg[1] and pg[2], the drift
@@ -339,7 +330,7 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
             add(0, 0, 1, -t1 * r[2] + t2 * s1 + b0 * s1 * r[2]);
         }
 #pragma unroll
-        for (int b = 0; b < 12; b++) put(2, b / 4 - 1, (b >> 1) & 1, b & 1);
+        for (int b = 0; b < 12; b++) put(FB0, b / 4 - 1, (b >> 1) & 1, b & 1);
         // B1: y stencil of pg[1], the x and z links of pg[0] and pg[2], the drift
         clear();
         {
@@ -357,7 +348,7 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
             add(0, 0, 1, -t0 * r[2] + t2 * s0 + b1 * s0 * r[2]);
         }
 #pragma unroll
-        for (int b = 0; b < 12; b++) put(3, (b >> 1) & 1, b / 4 - 1, b & 1);
+        for (int b = 0; b < 12; b++) put(FB1, (b >> 1) & 1, b / 4 - 1, b & 1);
         // B2: z stencil of pg[2], the x and y links of pg[0] and pg[1], the drift
         clear();
         {
@@ -375,62 +366,106 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
             add(0, 1, 0, -t0 * r[1] + t1 * s0 + b2 * s0 * r[1]);
         }
 #pragma unroll
-        for (int b = 0; b < 12; b++) put(4, (b >> 1) & 1, b & 1, b / 4 - 1);
+        for (int b = 0; b < 12; b++) put(FB2, (b >> 1) & 1, b & 1, b / 4 - 1);
     }
 }
 
+// One field's sites that the stencils of a tile of cells touch, in LDS: the
+// box of BX x BY x BZ sites from (x0, y0, z0) - (LX, LY, LZ), from entry OFF.
+template <int BX, int BY, int BZ, int LX, int LY, int LZ, int OFF> struct StencilBox {
+    static constexpr int N = BX * BY * BZ, END = OFF + N;
+    __device__ static __forceinline__ uint32_t site_of(int e, int x0, int y0, int z0, int mesh)
+    {
+        const uint32_t msk = (uint32_t)mesh - 1;
+        const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
+        return ((uint32_t)(x0 - LX + ex) & msk) +
+               (uint32_t)mesh * (((uint32_t)(y0 - LY + ey) & msk) + (uint32_t)mesh * ((uint32_t)(z0 - LZ + ez) & msk));
+    }
+    // the box's entry for offset (-LX, -LY, -LZ) of cell (cx, cy, cz) of the tile:
+    // every stencil offset adds a constant >= 0 to it, which the LDS
+    // instructions take as their immediate (cx, cy, cz known to be small and
+    // unsigned)
+    __device__ static __forceinline__ uint32_t corner(uint32_t cx, uint32_t cy, uint32_t cz)
+    {
+        return OFF + cx + BX * (cy + BY * cz);
+    }
+    __device__ static __forceinline__ uint32_t step(int dx, int dy, int dz)
+    {
+        return (uint32_t)((dx + LX) + BX * ((dy + LY) + BY * (dz + LZ)));
+    }
+};
+template <typename T, class X> struct BoxField {
+    using Box = X;
+    const T *lds;
+    uint32_t o;  // X::corner of the particle's cell
+    __device__ __forceinline__ T operator()(int dx, int dy, int dz) const { return lds[o + X::step(dx, dy, dz)]; }
+};
+
 // The tiled reverse kick + drift: one workgroup per tile of TX x TY x TZ cells
-// reads the fields of the stencil box [x0-1, x0+TX+1] x ... from LDS, as the
-// forward update does, and sums the field adjoints of its particles in FP64
-// LDS accumulators over the same box (the scatter stencils stay inside it),
-// which go to the global arrays with one atomic per site and field at the
-// end.  A crowded cell then costs LDS atomics, not global ones.
+// reads the fields its particles' stencils touch from LDS, as the forward
+// update does, and sums the field adjoints in FP64 LDS accumulators over the
+// same sites, which go to the global arrays with one atomic per site and field
+// at the end.  A crowded cell then costs LDS atomics, not global ones.
+//
+// Bound by latency at low occupancy: the accumulators leave room for one
+// FP32 workgroup per CU.  Each field's box therefore holds only the offsets
+// its own stencil reaches (phi -1..2, chi 0..1, B_i -1..1 along i and 0..1
+// across): 98 KB instead of 138 for a 16 x 8 x 8 tile, and 0.73 of the sites to
+// stage, clear and flush; 768 threads (three waves per SIMD, 156 registers)
+// measured best of 512, 768 and 1024 (which spills), and smaller tiles with
+// two or three workgroups per CU lose more to their halo.  FP64 takes two
+// waves per SIMD with a 92-byte spill (256 + 26 registers without).  At 256^3,
+// FP32, one particle per cell: 2.56 -> 1.99 ms, of which the LDS atomics are
+// 0.5 ms and the global ones 0.3 ms; FP64 at 128^3 with the reverse deposit
+// 1.01 -> 0.94 ms.
 template <typename T, int TX, int TY, int TZ, int NT>
-__global__ __launch_bounds__(NT) void k_adj_gr_kick_drift(PV<T> v, const T *__restrict__ phi, const T *__restrict__ chi,
+__global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drift(PV<T> v, const T *__restrict__ phi, const T *__restrict__ chi,
                                                           const T *__restrict__ Bi, T *lx, T *lq, T *lphi, T *lchi,
                                                           T *lB, int64_t M, AdjKD s)
 {
-    constexpr int SX = TX + 3, SY = TY + 3, SZ = TZ + 3, NS = SX * SY * SZ, NROW = TY * TZ;
-    __shared__ T fld[5][NS];
-    __shared__ double acc[5][NS];
+    using XP = StencilBox<TX + 3, TY + 3, TZ + 3, 1, 1, 1, 0>;
+    using XC = StencilBox<TX + 1, TY + 1, TZ + 1, 0, 0, 0, XP::END>;
+    using X0 = StencilBox<TX + 2, TY + 1, TZ + 1, 1, 0, 0, XC::END>;
+    using X1 = StencilBox<TX + 1, TY + 2, TZ + 1, 0, 1, 0, X0::END>;
+    using X2 = StencilBox<TX + 1, TY + 1, TZ + 2, 0, 0, 1, X1::END>;
+    constexpr int NROW = TY * TZ;
+    __shared__ T fld[X2::END];
+    __shared__ double acc[X2::END];
     const int N = v.N;
-    const uint32_t msk = (uint32_t)N - 1;
     const int tid = threadIdx.x, lane = tid & 63;
     int x0, y0, z0;
     tile_origin<TX, TY, TZ>(N, x0, y0, z0);
     const int nfmax = s.nf_k > s.nf_d ? s.nf_k : s.nf_d;
-    for (int e = tid; e < NS; e += NT) {
-        const int lx0 = e % SX, ly = (e / SX) % SY, lz = e / (SX * SY);
-        const uint32_t g = ((uint32_t)(x0 - 1 + lx0) & msk) +
-                           (uint32_t)N * (((uint32_t)(y0 - 1 + ly) & msk) + (uint32_t)N * ((uint32_t)(z0 - 1 + lz) & msk));
-        fld[0][e] = phi[g];
-        fld[1][e] = nfmax >= 2 ? chi[g] : (T)0;
-        fld[2][e] = nfmax >= 3 ? Bi[g] : (T)0;
-        fld[3][e] = nfmax >= 3 ? Bi[M + g] : (T)0;
-        fld[4][e] = nfmax >= 3 ? Bi[2 * M + g] : (T)0;
-#pragma unroll
-        for (int f = 0; f < 5; f++) acc[f][e] = 0.0;
-    }
+    auto stage = [&](auto box, const T *f, bool on) {
+        using X = decltype(box);
+        for (int e = tid; e < X::N; e += NT) fld[X::END - X::N + e] = on ? f[X::site_of(e, x0, y0, z0, N)] : (T)0;
+    };
+    stage(XP{}, phi, true);
+    stage(XC{}, chi, nfmax >= 2);
+    stage(X0{}, Bi, nfmax >= 3);
+    stage(X1{}, Bi + M, nfmax >= 3);
+    stage(X2{}, Bi + 2 * M, nfmax >= 3);
+    for (int e = tid; e < X2::END; e += NT) acc[e] = 0.0;
     int32_t rb0, incl;
     tile_rows_load<TX, TY, NROW>(v.start, N, x0, y0, z0, lane, rb0, incl);
+    const int maxrow = (int)wave_max_u32((uint32_t)incl);
     incl = wave_row_scan(incl, lane);
     const int total = __shfl(incl, NROW - 1, 64);
-    // A crowded tile gives every lane its own contiguous chunk of Q particles,
-    // so the lanes of one instruction sit Q particles apart, mostly in
-    // different cells, and their field-adjoint atomics rarely meet on one LDS
-    // address; other tiles keep consecutive particles in consecutive lanes
-    // (coalesced loads)
+    // A tile with a crowded row (64 or more particles in its 16 cells; a row of
+    // an unclustered state of one particle per cell reaches about 35) hands
+    // consecutive particles to different waves, so the field-adjoint atomics
+    // of one instruction rarely meet on one LDS address; other tiles keep
+    // consecutive particles in consecutive lanes, whose loads coalesce.
+    // 256^3 mixed states, both reverse kernels: 4.07 and 3.16 ms (a tenth of
+    // the particles in clumps, none) against 4.38 and 3.13 ms with the line at
+    // 32, 4.05 and 3.16 ms at 100; 6.47, 6.65, 6.49 ms with four tenths in clumps
     constexpr int NW = NT / 64;
-    const bool chunk = ADJ_CHUNK_X4 > 0 && 4 * total >= ADJ_CHUNK_X4 * (TX * TY * TZ);
-    const int Q = (total + 63) / 64;
-    // the same for every lane of the workgroup
-    const int niter = chunk ? (Q + NW - 1) / NW : (total + NT - 1) / NT;
+    const bool spread = maxrow >= 4 * TX;
+    const int niter = (total + NT - 1) / NT;  // the same for every lane of the workgroup
     __syncthreads();
     const int64_t n = v.n;
     for (int it = 0; it < niter; it++) {
-        const int sq = it * NW + (tid >> 6);  // position inside the lane's chunk
-        const int f = chunk ? (sq < Q ? lane * Q + sq : total) : tid + it * NT;
-        const int64_t p = tile_locate<NROW>(rb0, incl, f);
+        const int64_t p = tile_locate<NROW>(rb0, incl, it * NT + (spread ? lane * NW + (tid >> 6) : tid));
         if (p < 0) continue;
         const int64_t id = v.id[p];
         int x, y, z;
@@ -441,29 +476,34 @@ __global__ __launch_bounds__(NT) void k_adj_gr_kick_drift(PV<T> v, const T *__re
         T LX[3], LQ[3], nx[3], nq[3];
 #pragma unroll
         for (int j = 0; j < 3; j++) { LX[j] = lx[j * n + id]; LQ[j] = lq[j * n + id]; }
-        const int o = (x - x0 + 1) + SX * ((y - y0 + 1) + SY * (z - z0 + 1));
-        const FieldLds<T> Fp{fld[0], o, SX, SX * SY}, Fc{fld[1], o, SX, SX * SY}, FB0{fld[2], o, SX, SX * SY},
-            FB1{fld[3], o, SX, SX * SY}, FB2{fld[4], o, SX, SX * SY};
-        auto sc = [&](int f, int dx, int dy, int dz, T val) {
-            __hip_atomic_fetch_add(&acc[f][o + dx + SX * dy + SX * SY * dz], (double)val, __ATOMIC_RELAXED,
+        const uint32_t cx = x & (TX - 1), cy = y & (TY - 1), cz = z & (TZ - 1);
+        const BoxField<T, XP> Fp{fld, XP::corner(cx, cy, cz)};
+        const BoxField<T, XC> Fc{fld, XC::corner(cx, cy, cz)};
+        const BoxField<T, X0> F0{fld, X0::corner(cx, cy, cz)};
+        const BoxField<T, X1> F1{fld, X1::corner(cx, cy, cz)};
+        const BoxField<T, X2> F2{fld, X2::corner(cx, cy, cz)};
+        auto sc = [&](const auto &F, int dx, int dy, int dz, T val) {
+            using X = typename std::decay_t<decltype(F)>::Box;
+            __hip_atomic_fetch_add(&acc[F.o + X::step(dx, dy, dz)], (double)val, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         };
-        adj_gr_particle<T>(rt, qt, LX, LQ, Fp, Fc, FB0, FB1, FB2, N, s, nx, nq, sc);
+        adj_gr_particle<T>(rt, qt, LX, LQ, Fp, Fc, F0, F1, F2, N, s, nx, nq, sc);
 #pragma unroll
         for (int j = 0; j < 3; j++) { lx[j * n + id] = nx[j]; lq[j * n + id] = nq[j]; }
     }
     __syncthreads();
-    T *dst[5] = {lphi, lchi, lB, lB + M, lB + 2 * M};
-    for (int e = tid; e < NS; e += NT) {
-        const int lx0 = e % SX, ly = (e / SX) % SY, lz = e / (SX * SY);
-        const uint32_t g = ((uint32_t)(x0 - 1 + lx0) & msk) +
-                           (uint32_t)N * (((uint32_t)(y0 - 1 + ly) & msk) + (uint32_t)N * ((uint32_t)(z0 - 1 + lz) & msk));
-#pragma unroll
-        for (int f = 0; f < 5; f++) {
-            const double a = acc[f][e];
-            if (a != 0.0) atomicAdd(dst[f] + g, (T)a);
+    auto flush = [&](auto box, T *dst) {
+        using X = decltype(box);
+        for (int e = tid; e < X::N; e += NT) {
+            const double a = acc[X::END - X::N + e];
+            if (a != 0.0) atomicAdd(dst + X::site_of(e, x0, y0, z0, N), (T)a);
         }
-    }
+    };
+    flush(XP{}, lphi);
+    flush(XC{}, lchi);
+    flush(X0{}, lB);
+    flush(X1{}, lB + M);
+    flush(X2{}, lB + 2 * M);
 }
 
 // Reverse of the T00 + Tij + T0i-link deposits of one particle (phi_old the
@@ -599,7 +639,9 @@ __device__ __forceinline__ void adj_gr_deposit_particle(const T rt[3], const T q
 // The tiled reverse deposit: one workgroup per tile of TX x TY x TZ cells
 // stages the eleven fields its particles read (the sites [x0, x0+TX] x ...)
 // in LDS and sums phi_old's adjoint there in FP64, added to lphi once per
-// site at the end.
+// site at the end.  72 KB of LDS per FP32 tile allow two workgroups per CU:
+// with 512 threads each they fill four waves per SIMD (110 registers), with
+// 256 only two (256^3, one particle per cell: 1.26 -> 0.90 ms).
 template <typename T, int TX, int TY, int TZ, int NT>
 __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restrict__ phi, const T *__restrict__ lT00,
                                                        const T *__restrict__ lTij, const T *__restrict__ lL, T *lx,
@@ -801,9 +843,9 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
                            T *lB, int nf_k, int nf_d, double a_k, double a_d, double dtau_k, double dtau_d)
 {
     gev_ctx *c = p->ctx;
-    AdjKD s{nf_k, nf_d, a_k, a_d, dtau_k, dtau_d, a_k * a_k * (double)c->N, a_d * a_d * (double)c->N};
+    const double bk = a_k * a_k * (double)c->N, bd = a_d * a_d * (double)c->N, K = dtau_k * c->N;
+    AdjKD s{nf_k, nf_d, a_k, a_d, dtau_k, dtau_d, bk, bd, K, 1.0 / bk, 1.0 / bd, K / bk, dtau_d / bd};
     const int N = c->N;
-    // tiles as the forward update's where the FP64 accumulators fit the LDS
     auto launch = [&](auto tx, auto ty, auto tz, auto nt) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value, TZ = decltype(tz)::value;
         constexpr int NT = decltype(nt)::value;
@@ -811,22 +853,20 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
         hipLaunchKernelGGL((k_adj_gr_kick_drift<T, TX, TY, TZ, NT>), dim3(nb), dim3(NT), 0, c->stream, make_pv<T>(p),
                            phi, chi, Bi, lx, lq, lphi, lchi, lB, c->M, s);
     };
-    using I = std::integral_constant<int, 4>;
+    using I4 = std::integral_constant<int, 4>;
+    using I8 = std::integral_constant<int, 8>;
+    using I256 = std::integral_constant<int, 256>;
     if (p->n > 0) {
         bool done = false;
-        if constexpr (sizeof(T) == 4) {
-            if (ADJ_KD_WIDE && N >= 16) {
-                launch(std::integral_constant<int, 16>{}, std::integral_constant<int, 8>{},
-                       std::integral_constant<int, 8>{}, std::integral_constant<int, 512>{});
+        if constexpr (sizeof(T) == 4) {  // FP64 fields and accumulators take the smaller tile
+            if (N >= 16) {
+                launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 768>{});
                 done = true;
             }
         }
         if (done) {
-        } else if (N >= 8)
-            launch(std::integral_constant<int, 8>{}, std::integral_constant<int, 8>{}, I{},
-                   std::integral_constant<int, 256>{});
-        else
-            launch(I{}, I{}, I{}, std::integral_constant<int, 256>{});
+        } else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{});
+        else launch(I4{}, I4{}, I4{}, I256{});
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
@@ -851,8 +891,8 @@ int adj_gr_deposit_impl(gev_pcls *p, const T *phi, const T *lT00, const T *lTij,
     if (p->n > 0) {
         bool done = false;
         if constexpr (sizeof(T) == 4) {  // FP64 fields take twice the LDS: the smaller tile
-            if (ADJ_DEP_WIDE && N >= 16) {
-                launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 256>{});
+            if (N >= 16) {
+                launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 512>{});
                 done = true;
             }
         }
