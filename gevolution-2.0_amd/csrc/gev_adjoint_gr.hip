@@ -21,6 +21,7 @@
 // order follows atomic arbitration).  Per-particle adjoints lx, lq are [3][n]
 // arrays indexed by particle ID, as in the Newtonian adjoint; positions in box
 // units (d/dx = N d/dr).
+#include <array>
 #include <type_traits>
 
 #include "gev_common.hpp"
@@ -414,10 +415,9 @@ template <typename T, class X> struct BoxField {
 // stage, clear and flush; 768 threads (three waves per SIMD, 156 registers)
 // measured best of 512, 768 and 1024 (which spills), and smaller tiles with
 // two or three workgroups per CU lose more to their halo.  FP64 takes two
-// waves per SIMD with a 92-byte spill (256 + 26 registers without).  At 256^3,
-// FP32, one particle per cell: 2.56 -> 1.99 ms, of which the LDS atomics are
-// 0.5 ms and the global ones 0.3 ms; FP64 at 128^3 with the reverse deposit
-// 1.01 -> 0.94 ms.
+// waves per SIMD with a 12-byte spill.  At 256^3, FP32, one particle per cell:
+// 2.56 -> 1.8 ms, of which the LDS atomics are 0.5 ms and the global ones
+// 0.3 ms; FP64 at 128^3 with the reverse deposit 1.01 -> 0.77 ms.
 template <typename T, int TX, int TY, int TZ, int NT>
 __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drift(PV<T> v, const T *__restrict__ phi, const T *__restrict__ chi,
                                                           const T *__restrict__ Bi, T *lx, T *lq, T *lphi, T *lchi,
@@ -436,15 +436,37 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
     int x0, y0, z0;
     tile_origin<TX, TY, TZ>(N, x0, y0, z0);
     const int nfmax = s.nf_k > s.nf_d ? s.nf_k : s.nf_d;
-    auto stage = [&](auto box, const T *f, bool on) {
+    // all of a thread's field loads are requested before the first LDS write
+    auto load = [&](auto box, const T *f, bool on) {
         using X = decltype(box);
-        for (int e = tid; e < X::N; e += NT) fld[X::END - X::N + e] = on ? f[X::site_of(e, x0, y0, z0, N)] : (T)0;
+        std::array<T, (X::N + NT - 1) / NT> t;
+#pragma unroll
+        for (int k = 0; k < (int)t.size(); k++) {
+            const int e = tid + k * NT;
+            t[k] = on && e < X::N ? f[X::site_of(e, x0, y0, z0, N)] : (T)0;
+        }
+        return t;
     };
-    stage(XP{}, phi, true);
-    stage(XC{}, chi, nfmax >= 2);
-    stage(X0{}, Bi, nfmax >= 3);
-    stage(X1{}, Bi + M, nfmax >= 3);
-    stage(X2{}, Bi + 2 * M, nfmax >= 3);
+    auto put = [&](auto box, const auto &t) {
+        using X = decltype(box);
+#pragma unroll
+        for (int k = 0; k < (int)t.size(); k++) {
+            const int e = tid + k * NT;
+            if (e < X::N) fld[X::END - X::N + e] = t[k];
+        }
+    };
+    {
+        const auto tp = load(XP{}, phi, true);
+        const auto tc = load(XC{}, chi, nfmax >= 2);
+        const auto t0 = load(X0{}, Bi, nfmax >= 3);
+        const auto t1 = load(X1{}, Bi + M, nfmax >= 3);
+        const auto t2 = load(X2{}, Bi + 2 * M, nfmax >= 3);
+        put(XP{}, tp);
+        put(XC{}, tc);
+        put(X0{}, t0);
+        put(X1{}, t1);
+        put(X2{}, t2);
+    }
     for (int e = tid; e < X2::END; e += NT) acc[e] = 0.0;
     int32_t rb0, incl;
     tile_rows_load<TX, TY, NROW>(v.start, N, x0, y0, z0, lane, rb0, incl);
@@ -456,9 +478,10 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
     // consecutive particles to different waves, so the field-adjoint atomics
     // of one instruction rarely meet on one LDS address; other tiles keep
     // consecutive particles in consecutive lanes, whose loads coalesce.
-    // 256^3 mixed states, both reverse kernels: 4.07 and 3.16 ms (a tenth of
-    // the particles in clumps, none) against 4.38 and 3.13 ms with the line at
-    // 32, 4.05 and 3.16 ms at 100; 6.47, 6.65, 6.49 ms with four tenths in clumps
+    // 256^3 mixed states, both reverse kernels (measured before the loads were
+    // requested together): 4.07 and 3.16 ms (a tenth of the particles in
+    // clumps, none) against 4.38 and 3.13 ms with the line at 32, 4.05 and
+    // 3.16 ms at 100; 6.47, 6.65, 6.49 ms with four tenths in clumps
     constexpr int NW = NT / 64;
     const bool spread = maxrow >= 4 * TX;
     const int niter = (total + NT - 1) / NT;  // the same for every lane of the workgroup
@@ -858,8 +881,12 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
     using I256 = std::integral_constant<int, 256>;
     if (p->n > 0) {
         bool done = false;
-        if constexpr (sizeof(T) == 4) {  // FP64 fields and accumulators take the smaller tile
-            if (N >= 16) {
+        if constexpr (sizeof(T) == 4) {
+            // FP64 fields and accumulators take the smaller tile, and so do
+            // meshes whose large tiles would leave CUs idle (both reverse
+            // kernels at 32^3: 57 against 94 us with 32 large tiles; at 64^3,
+            // 256 large tiles, 137 against 150 us)
+            if (N >= 64) {
                 launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 768>{});
                 done = true;
             }
@@ -890,8 +917,8 @@ int adj_gr_deposit_impl(gev_pcls *p, const T *phi, const T *lT00, const T *lTij,
     using I8 = std::integral_constant<int, 8>;
     if (p->n > 0) {
         bool done = false;
-        if constexpr (sizeof(T) == 4) {  // FP64 fields take twice the LDS: the smaller tile
-            if (N >= 16) {
+        if constexpr (sizeof(T) == 4) {  // FP64 fields take twice the LDS: the smaller tile; N as above
+            if (N >= 64) {
                 launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 512>{});
                 done = true;
             }

@@ -2,7 +2,7 @@
 // passes: x (real<->half-complex, contiguous lines), then y and z (complex,
 // strided columns read as TX-wide coalesced row segments).  Radix-8/4/2
 // Stockham stages in LDS, twiddles from a per-size table in global memory.
-// For 16 <= N <= 128 the x and y passes are one kernel per plane
+// For 16 <= N <= 128 (FP64: 64) the x and y passes are one kernel per plane
 // (gev_fft_plane.hpp), all components of a field in one launch.
 #include <algorithm>
 #include <type_traits>
@@ -487,10 +487,10 @@ static void launch_r2c_src(const Src &src, cx<T> *out, int P, int64_t nlines, co
 template <typename T, int N>
 static void launch_r2c(const T *in, cx<T> *out, int P, int64_t nlines, const cx<T> *tw, hipStream_t s)
 {
-    if constexpr (N >= 256) {
+    if constexpr (N >= 128) {
         launch_r2c_src<T, N>(SrcPlain<T, N>{in}, out, P, nlines, tw, s);
     } else {
-        static_assert(N <= 8, "16 <= N <= 128 transforms whole planes");
+        static_assert(N <= 8, "16 <= N <= 64 transforms whole planes");
         constexpr int NLINES = 4096 / N > 1024 ? 1024 : 4096 / N;
         int64_t nb = (nlines + NLINES - 1) / NLINES;
         hipLaunchKernelGGL((k_r2c_x<T, N, NLINES>), dim3((unsigned)nb), dim3(FFT_NT), 0, s, in, out, P, nlines, tw);
@@ -500,13 +500,13 @@ static void launch_r2c(const T *in, cx<T> *out, int P, int64_t nlines, const cx<
 template <typename T, int N>
 static void launch_c2r(const cx<T> *in, T *out, int P, int64_t nlines, const cx<T> *tw, hipStream_t s)
 {
-    if constexpr (N >= 256) {
+    if constexpr (N >= 128) {
         constexpr int NL = xlines<T, N>();
         int64_t nb = (nlines + NL - 1) / NL;
         hipLaunchKernelGGL((k_c2r_x_reg<T, N, NL>), dim3((unsigned)nb), dim3(NL * N / 16), 0, s, in, out, P, nlines,
                            tw);
     } else {
-        static_assert(N <= 8, "16 <= N <= 128 transforms whole planes");
+        static_assert(N <= 8, "16 <= N <= 64 transforms whole planes");
         constexpr int NLINES = 4096 / N > 1024 ? 1024 : 4096 / N;
         int64_t nb = (nlines + NLINES - 1) / NLINES;
         hipLaunchKernelGGL((k_c2r_x<T, N, NLINES>), dim3((unsigned)nb), dim3(FFT_NT), 0, s, in, out, P, nlines, tw);
@@ -537,7 +537,10 @@ template <typename T, int N> struct CompPlain {
     template <class F> __device__ __forceinline__ void with(int c, F f) const { f(SrcPlain<T, N>{in + c * M}); }
 };
 
-constexpr bool plane_size(int N) { return N >= 16 && N <= 128; }
+// FP64 planes of N = 128 fill the LDS (one workgroup per CU, 64 to 128 of the
+// 256 CUs) and lose to the separate passes: 128^3 FP64 GR cycles 936 against
+// 903 us each; FP32 ones gain (see gev_fft_plane.hpp)
+template <typename T> constexpr bool plane_size(int N) { return N >= 16 && (N <= 64 || (N == 128 && sizeof(T) == 4)); }
 
 // forward x and y passes of ncomp components (r2c without the z pass) from
 // plane sources, and the inverse y and x passes
@@ -550,7 +553,7 @@ static void launch_fwd_plane(gev_ctx *c, const Comp &comp, cx<T> *out, int ncomp
 }
 template <typename T, int N> static void fwd_xy(gev_ctx *c, const T *in, cx<T> *out, int ncomp, const cx<T> *tw)
 {
-    if constexpr (plane_size(N)) {
+    if constexpr (plane_size<T>(N)) {
         launch_fwd_plane<T, N>(c, CompPlain<T, N>{in, c->M}, out, ncomp, tw);
     } else {
         for (int i = 0; i < ncomp; i++) {
@@ -561,7 +564,7 @@ template <typename T, int N> static void fwd_xy(gev_ctx *c, const T *in, cx<T> *
 }
 template <typename T, int N> static void inv_yx(gev_ctx *c, cx<T> *in, T *out, int ncomp, const cx<T> *tw)
 {
-    if constexpr (plane_size(N)) {
+    if constexpr (plane_size<T>(N)) {
         hipLaunchKernelGGL((k_inv_plane<T, N>), dim3(N / plane_np<N>(), ncomp), dim3(plane_nt<N>()), 0, c->stream, in,
                            out, c->NK, c->M, tw);
     } else {
@@ -578,7 +581,7 @@ template <typename T, int N> static void inv_yx(gev_ctx *c, cx<T> *in, T *out, i
 // components at a time: all of them where a component is small (launches and
 // latency count); one by one on large meshes, whose passes then find the
 // component just written in the Infinity Cache
-template <int N> constexpr int fft_batch() { return plane_size(N) ? 64 : 1; }
+template <typename T, int N> constexpr int fft_batch() { return plane_size<T>(N) ? 64 : 1; }
 
 template <typename T>
 int fft_r2c_impl(gev_ctx *ctx, const T *in, cx<T> *out, int ncomp, const cx<T> *tw)
@@ -587,8 +590,8 @@ int fft_r2c_impl(gev_ctx *ctx, const T *in, cx<T> *out, int ncomp, const cx<T> *
     switch (ctx->N) {
 #define X(n)                                                                        \
     case n:                                                                         \
-        for (int c = 0; c < ncomp; c += fft_batch<n>()) {                           \
-            const int m = std::min(ncomp - c, fft_batch<n>());                      \
+        for (int c = 0; c < ncomp; c += fft_batch<T, n>()) {                           \
+            const int m = std::min(ncomp - c, fft_batch<T, n>());                      \
             fwd_xy<T, n>(ctx, in + c * M, out + c * NK, m, tw);                     \
             launch_col<T, n>(out + c * NK, ctx->P, 2, -1, tw, ctx->stream, m);      \
         }                                                                           \
@@ -608,8 +611,8 @@ int fft_c2r_impl(gev_ctx *ctx, cx<T> *in, T *out, int ncomp, const cx<T> *tw)
     switch (ctx->N) {
 #define X(n)                                                                        \
     case n:                                                                         \
-        for (int c = 0; c < ncomp; c += fft_batch<n>()) {                           \
-            const int m = std::min(ncomp - c, fft_batch<n>());                      \
+        for (int c = 0; c < ncomp; c += fft_batch<T, n>()) {                           \
+            const int m = std::min(ncomp - c, fft_batch<T, n>());                      \
             launch_col<T, n>(in + c * NK, ctx->P, 2, +1, tw, ctx->stream, m);       \
             inv_yx<T, n>(ctx, in + c * NK, out + c * M, m, tw);                     \
         }                                                                           \
@@ -998,9 +1001,9 @@ static void zsolve_chain(gev_ctx *c, int op, const T *rin, int nin, cx<T> *ftin,
                          const ZParams &zp)
 {
     const cx<T> *tw = twiddles_of<T>(c);
-    if (op == ZOP_SCALAR && !plane_size(N)) {
+    if (op == ZOP_SCALAR && !plane_size<T>(N)) {
         // x passes, then the y pass that forms the three groups of projectFTscalar
-        if constexpr (!plane_size(N)) {
+        if constexpr (!plane_size<T>(N)) {
             for (int i = 0; i < nin; i++)
                 launch_r2c<T, N>(rin + i * c->M, ftin + i * c->NK, c->P, (int64_t)N * N, tw, c->stream);
             launch_col_comb<T, N>(ftin, c->P, c->NK, tw, zp, c->stream);
@@ -1012,7 +1015,7 @@ static void zsolve_chain(gev_ctx *c, int op, const T *rin, int nin, cx<T> *ftin,
             launch_zsolve<T, N, ZOP_POISSON>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
         else if (op == ZOP_VECTOR)
             launch_zsolve<T, N, ZOP_VECTOR>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
-        else if constexpr (plane_size(N))
+        else if constexpr (plane_size<T>(N))
             launch_zsolve<T, N, ZOP_SCALAR>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
     }
     inv_yx<T, N>(c, ftout, rout, nout, tw);
@@ -1078,7 +1081,7 @@ static void poisson_T00_chain(gev_ctx *c, const SrcT00<T, N> &src, T *put, T *po
     const cx<T> *tw = twiddles_of<T>(c);
     zp.parts = c->red + 64;
     zp.sums = c->red;
-    if constexpr (plane_size(N)) {
+    if constexpr (plane_size<T>(N)) {
         zp.nparts = N / plane_np<N>();
         launch_fwd_plane<T, N>(c, CompT00<T, N>{src, put}, work, 1, tw, c->red + 64);
     } else {
@@ -1151,7 +1154,7 @@ static void chi_from_Tij_chain(gev_ctx *c, const T *phi, T *Tij, T coeff, cx<T> 
     const int64_t nl = (int64_t)N * N;
     const cx<T> *tw = twiddles_of<T>(c);
     ZParams zp{c->gk2, c->kshift, 0.0, 0.0, 0.0, 0.0, 0, nullptr, 0, nullptr};
-    if constexpr (plane_size(N)) {
+    if constexpr (plane_size<T>(N)) {
         launch_fwd_plane<T, N>(c, CompSij<T, N>{phi, Tij, c->M, coeff}, SijFT, 6, tw);
         launch_zsolve<T, N, ZOP_SCALAR>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
     } else {
@@ -1200,7 +1203,7 @@ template <typename T, int N>
 static void vector_from_links_chain(gev_ctx *c, T *Bi, const T *phi, cx<T> *BiFT, const ZParams &zp)
 {
     const cx<T> *tw = twiddles_of<T>(c);
-    if constexpr (plane_size(N)) {
+    if constexpr (plane_size<T>(N)) {
         launch_fwd_plane<T, N>(c, CompLink<T, N>{phi, Bi, c->M}, BiFT, 3, tw);
     } else {
         const int64_t nl = (int64_t)N * N, M = c->M;

@@ -1,8 +1,8 @@
 // gev_fft_plane.hpp -- x and y transforms of a whole z plane in one workgroup
-// (16 <= N <= 128).
+// (16 <= N <= 128 in FP32, up to 64 in FP64).
 //
-// Up to N = 128 the half spectrum of a plane fits the LDS of one workgroup
-// (N (N/2 + 1) complex values: 66 KB in FP32 and 133 KB in FP64 at N = 128),
+// The half spectrum of such a plane fits the LDS with room for a second
+// workgroup (N (N/2 + 1) complex values: 66 KB at N = 128 in FP32),
 // so the plane is read once, transformed along x and along y in LDS and
 // written once; all components of a field go in one launch.  At these sizes
 // the transforms are bound by launches and by the latency of each pass, not by

@@ -23,7 +23,7 @@ def gp():
     return gevpm
 
 
-@pytest.mark.parametrize("prec,N,n,nf", [("mixed", 16, 1500, 3), ("mixed", 32, 2111, 3), ("mixed", 16, 777, 2),
+@pytest.mark.parametrize("prec,N,n,nf", [("mixed", 16, 1500, 3), ("mixed", 32, 2111, 3), ("mixed", 64, 3001, 3), ("mixed", 16, 777, 2),
                                          ("fp64", 16, 1000, 3), ("fp64", 8, 401, 3), ("mixed", 8, 401, 3)])
 def test_crowded_rows_match_sparse_ones(gp, prec, N, n, nf):
     ctx = gp.Context(N, gp.GEV_FP64 if prec == "fp64" else gp.GEV_MIXED)
