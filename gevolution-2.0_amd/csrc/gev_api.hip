@@ -662,6 +662,21 @@ int gev_adj_project_ft_scalar(gev_ctx *c, const void *lchiFT, void *lSijFT)
                          adj_project_ft_scalar_impl<float>(c, (const cx<float> *)lchiFT, (cx<float> *)lSijFT));
 }
 
+int gev_adj_solve_chi(gev_ctx *c, const void *lchi, void *lSij, void *chiFT, void *SijFT)
+{
+    CHECK(c && lchi && lSij && chiFT && SijFT, "gev_adj_solve_chi: NULL argument");
+    if (zsolve_supported(c))
+        return PREC_DISPATCH(c,
+                             adj_solve_chi_fused_impl<double>(c, (const double *)lchi, (double *)lSij,
+                                                              (cx<double> *)chiFT, (cx<double> *)SijFT),
+                             adj_solve_chi_fused_impl<float>(c, (const float *)lchi, (float *)lSij, (cx<float> *)chiFT,
+                                                             (cx<float> *)SijFT));
+    int rc = gev_fft_r2c(c, lchi, chiFT, 1);
+    if (!rc) rc = gev_adj_project_ft_scalar(c, chiFT, SijFT);
+    if (!rc) rc = gev_fft_c2r(c, SijFT, lSij, 6);
+    return rc;
+}
+
 // ---- fused real -> k-space -> real solves (the operator runs inside the z pass)
 int gev_solve_poisson(gev_ctx *c, const void *src, void *pot, void *workFT, double coeff, double modif, int set_k0,
                       double k0_re)

@@ -639,7 +639,9 @@ int fft_c2r_impl(gev_ctx *ctx, cx<T> *in, T *out, int ncomp, const cx<T> *tw)
 //   B = S_xx + S_yy - 2 S_zz,   C = -6 (k0 S_xz + k1 S_yz)
 // ZOP_SCALAR3: the same from the three groups that k_col_comb forms in the y
 // pass (below) instead of the six components
-enum { ZOP_POISSON = 0, ZOP_SCALAR = 1, ZOP_VECTOR = 2, ZOP_SCALAR3 = 3 };
+// ZOP_ADJ_SCALAR: projectFTscalar's adjoint, one component in and the six
+// conj(w_c) lchi / (2 k^4 N) out
+enum { ZOP_POISSON = 0, ZOP_SCALAR = 1, ZOP_VECTOR = 2, ZOP_SCALAR3 = 3, ZOP_ADJ_SCALAR = 4 };
 
 struct ZParams {
     const double *gk2;
@@ -895,6 +897,46 @@ __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(c
         inverse(0, std::integral_constant<int, 0>{});
         inverse(1, std::integral_constant<int, 1>{});
         inverse(2, std::integral_constant<int, 2>{});
+    } else if constexpr (OP == ZOP_ADJ_SCALAR) {
+        // the one forward transform stays in registers; every component's
+        // modes go through LDS to its inverse transform
+        __shared__ double gkd[L];
+        __shared__ cx<double> ksd[L];
+        for (int m = threadIdx.x; m < L; m += NT) {
+            gkd[m] = zp.gk2[m];
+            ksd[m] = zp.ks[m];
+        }
+        auto st = [&](int ln, int row, cx<T> v, int slot) {
+            lines[slot] = ln;
+            poss[slot] = row;
+            vin[0][slot] = v;
+        };
+        forward(std::integral_constant<int, 0>{}, st);
+        auto component = [&](auto cc) {
+            constexpr int C = decltype(cc)::value;
+            __syncthreads();  // previous transform done with lds
+#pragma unroll
+            for (int s = 0; s < 8; s++) {
+                const int kx = ct * TX + lines[s], kz = poss[s];
+                cx<double> r = mk(0.0, 0.0);
+                if (kx <= H && !(kx == 0 && ky == 0 && kz == 0)) {
+                    const cx<double> w = conj(kop_scalar_weight(C, gkd[kx], gy, gkd[kz], ksd[kx], kyv, ksd[kz]));
+                    r = (w * mk((double)vin[0][s].x, (double)vin[0][s].y)) * kop_scalar_norm(gkd[kx] + gy + gkd[kz], L);
+                }
+                lds[lines[s] * LDL + kz] = mk((T)r.x, (T)r.y);
+            }
+            __syncthreads();
+            cx<T> *dst = out + C * NK + off;
+            auto ld2 = [&](int line, int row) { return lds[line * LDL + row]; };
+            auto st2 = [&](int line, int row, cx<T> v, int) { dst[(int64_t)row * stride + line] = v; };
+            reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, +1, ld2, st2);
+        };
+        component(std::integral_constant<int, 0>{});
+        component(std::integral_constant<int, 1>{});
+        component(std::integral_constant<int, 2>{});
+        component(std::integral_constant<int, 3>{});
+        component(std::integral_constant<int, 4>{});
+        component(std::integral_constant<int, 5>{});
     } else {
         // chi = sum_c w_c S_c from the three kz groups:
         //   sum_c w_c S_c = FFT_z(A) + g2 FFT_z(B) + k2 FFT_z(C)
@@ -1180,6 +1222,34 @@ int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, T *Tij, double coeff, T *
     return GEV_OK;
 }
 
+// lS[c] = c2r(conj(w_c) r2c(lchi) / (2 k^4 N)): the adjoint of solve_chi.  The
+// weights are applied between the forward and the six inverse z transforms,
+// so no Fourier component passes through memory in between (the operator's
+// own kernel and six z passes before: at 128^3 FP32 13.7 + 44 us of the adjoint
+// chi solve)
+template <typename T, int N>
+static void adj_chi_chain(gev_ctx *c, const T *lchi, T *lS, cx<T> *work1, cx<T> *work6)
+{
+    const cx<T> *tw = twiddles_of<T>(c);
+    ZParams zp{c->gk2, c->kshift, 0.0, 0.0, 0.0, 0.0, 0, nullptr, 0, nullptr};
+    fwd_xy<T, N>(c, lchi, work1, 1, tw);
+    launch_zsolve<T, N, ZOP_ADJ_SCALAR>(work1, work6, c->P, c->NK, tw, zp, c->stream);
+    inv_yx<T, N>(c, work6, lS, 6, tw);
+}
+
+template <typename T>
+int adj_solve_chi_fused_impl(gev_ctx *c, const T *lchi, T *lS, cx<T> *work1, cx<T> *work6)
+{
+    switch (c->N) {
+#define X(n) case n: adj_chi_chain<T, n>(c, lchi, lS, work1, work6); break;
+        GEV_FOR_FUSED_N(X)
+#undef X
+    default: gev_set_error("the fused adjoint chi solve needs 16 <= N <= 1024"); return GEV_ERR_ARG;
+    }
+    GEV_HIP(hipGetLastError());
+    return GEV_OK;
+}
+
 // Bi = c2r(projectFTvector(r2c(Bi))), in place on Bi
 template <typename T> int solve_vector_fused_impl(gev_ctx *c, T *Bi, cx<T> *BiFT, double coeff, double modif)
 {
@@ -1258,6 +1328,7 @@ int solve_vector_links_fused_impl(gev_ctx *c, T *Bi, const T *phi, cx<T> *BiFT, 
     template int solve_chi_Tij_fused_impl<T>(gev_ctx *, const T *, T *, double, T *, cx<T> *, cx<T> *);  \
     template int solve_poisson_fused_impl<T>(gev_ctx *, const T *, T *, cx<T> *, double, double, int, double); \
     template int solve_chi_fused_impl<T>(gev_ctx *, const T *, T *, cx<T> *, cx<T> *);                  \
+    template int adj_solve_chi_fused_impl<T>(gev_ctx *, const T *, T *, cx<T> *, cx<T> *);               \
     template int solve_vector_fused_impl<T>(gev_ctx *, T *, cx<T> *, double, double);                    \
     template int solve_vector_links_fused_impl<T>(gev_ctx *, T *, const T *, cx<T> *, double, double);    \
     template int t0i_link_factor_impl<T>(gev_ctx *, T *, const T *);                                      \

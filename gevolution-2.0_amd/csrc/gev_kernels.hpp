@@ -32,6 +32,8 @@ template <typename T> int solve_chi_fused_impl(gev_ctx *c, const T *Sij, T *chi,
 // below N = 128 Tij is overwritten with Sij
 template <typename T>
 int solve_chi_Tij_fused_impl(gev_ctx *c, const T *phi, T *Tij, double coeff, T *chi, cx<T> *SijFT, cx<T> *chiFT);
+// the adjoint of solve_chi: lS (6) from lchi
+template <typename T> int adj_solve_chi_fused_impl(gev_ctx *c, const T *lchi, T *lS, cx<T> *work1, cx<T> *work6);
 template <typename T> int solve_vector_fused_impl(gev_ctx *c, T *Bi, cx<T> *BiFT, double coeff, double modif);
 // Bi holds T0i link sums (no 1 + phi_a + phi_b factor) on entry, B on return
 // (16 <= N <= 1024)

@@ -224,11 +224,13 @@ class Context:
         out = self.real_empty(6) if out is None else out
         work1 = self.fourier(1) if work1 is None else work1
         work6 = self.fourier(6) if work6 is None else work6
-        self.fft_r2c(lchi, out=work1)
+        lchi = lchi.contiguous()
+        nm = "adj_solve_chi"
         self.bind_stream()
-        check(lib.gev_adj_project_ft_scalar(self._h, self.k(work1, 1, "adj_solve_chi(work1)"),
-                                            self.k(work6, 6, "adj_solve_chi(work6)")), "gev_adj_project_ft_scalar")
-        return self.fft_c2r(work6, out=out, preserve=False)
+        check(lib.gev_adj_solve_chi(self._h, self.r(lchi, 1, nm + "(lchi)"), self.r(out, 6, nm + "(out)"),
+                                    self.k(work1, 1, nm + "(work1)"), self.k(work6, 6, nm + "(work6)")),
+              "gev_adj_solve_chi")
+        return out
 
     # ------------------------------------ fused real -> k -> real solves
     def solve_poisson(self, src, coeff, modif=0.0, k0=None, out=None, work=None):
@@ -242,10 +244,11 @@ class Context:
         return out
 
     def solve_poisson_T00(self, phi, chi, source, bg, c1, c2, c3, coeff, modif=0.0, k0set=False, out=None,
-                          work=None):
+                          work=None, want_sums=True):
         """prepareFTsource (T00 form) and the Poisson solve in one chain; returns
         (potential, (sum of source, sum of the source terms)).  source is only
-        read for 128 <= N <= 1024 and overwritten by the source terms below."""
+        read for 128 <= N <= 1024 and overwritten by the source terms below.
+        want_sums=False returns (potential, None) without waiting for the stream."""
         out = torch.empty_like(phi) if out is None else out
         work = self.fourier(1) if work is None else work
         sums = (C.c_double * 2)()
@@ -253,9 +256,9 @@ class Context:
         nm = "solve_poisson_T00"
         check(lib.gev_solve_poisson_T00(self._h, self.r(phi, 1, nm + "(phi)"), self.r(chi, 1, nm + "(chi)"),
                                         self.r(source, 1, nm + "(source)"), bg, c1, c2, c3, self.r(out, 1, nm + "(out)"),
-                                        self.k(work, 1, nm + "(work)", at_least=True), coeff, modif, int(k0set), sums),
-              "gev_solve_poisson_T00")
-        return out, (sums[0], sums[1])
+                                        self.k(work, 1, nm + "(work)", at_least=True), coeff, modif, int(k0set),
+                                        sums if want_sums else None), "gev_solve_poisson_T00")
+        return out, (sums[0], sums[1]) if want_sums else None
 
     def solve_chi(self, Sij, out=None, work6=None, work1=None):
         """c2r(projectFTscalar(r2c(Sij)))"""

@@ -187,7 +187,7 @@ class PMRunGR:
         self.dx = 1.0 / N
         self.phi, self.chi = c.real(1), c.real(1)
         self.T00, self.Tij, self.L = c.real(1), c.real(6), c.real(3)
-        self.src, self.Bi = c.real(1), c.real(3)
+        self.src = c.real(1) if N < 128 else None
         self.work1, self.work3, self.work6 = c.fourier(1), c.fourier(3), c.fourier(6)
         a = 1.0 / (1.0 + z_in)
         tau0 = particle_horizon(a, self.fpg, omega_m, omega_lambda)
@@ -223,10 +223,12 @@ class PMRunGR:
         self.Tij, self.L"""
         s, c, p, k_ = self.sched[k], self.ctx, self.pcls, self._coef(k)
         p.project_T00_Tij_T0i_links(self.T00, self.Tij, self.L, a=s["a"], phi=phi_old, coeff=1.0)
-        c.prepare_source_T00(phi_old, chi_old, self.T00, self.om, k_["c1"], k_["c2"], k_["c3"], result=self.src)
-        phi = c.solve_poisson(self.src, k_["pcoeff"], k_["modif"], work=self.work1)
-        Sij = c.prepare_source_Tij(phi, self.Tij, k_["ccoeff"])
-        chi = c.solve_chi(Sij, work6=self.work6, work1=self.work1)
+        # T00 and the links stay as they are for the reverse cycle: the phi
+        # solve forms its source in place below N = 128, so it gets a copy there
+        src = self.T00 if self.N >= 128 else self.src.copy_(self.T00)
+        phi, _ = c.solve_poisson_T00(phi_old, chi_old, src, self.om, k_["c1"], k_["c2"], k_["c3"], k_["pcoeff"],
+                                     k_["modif"], work=self.work1, want_sums=False)
+        chi = c.solve_chi_Tij(phi, self.Tij, k_["ccoeff"], work6=self.work6, work1=self.work1)
         B = self.L.clone()
         c.solve_vector_T0i_links(B, phi, k_["bcoeff"], 0.0, work=self.work3)
         return phi, chi, B

@@ -386,7 +386,9 @@ int gev_adj_ic_lattice(gev_ctx *ctx, const void *lx, const void *lq, double cx, 
  *      adjoint) and the link sums L (3): lphi += sum over links of L u at
  *      both ends; u is replaced by lL = (1 + phi_a + phi_b) u
  *   gev_adj_project_ft_scalar: k-space adjoint of projectFTscalar, lSijFT (6
- *      components) = conj(weights) lchiFT / (2 k^4 N) (overwritten) */
+ *      components) = conj(weights) lchiFT / (2 k^4 N) (overwritten)
+ *   gev_adj_solve_chi: the adjoint of gev_solve_chi, lSij (6, overwritten)
+ *      from lchi; chiFT (1) and SijFT (6) are work space */
 int gev_adj_gr_kick_drift(gev_pcls *p, const void *phi, const void *chi, const void *Bi, void *lx, void *lq,
                           void *lphi, void *lchi, void *lB, int nfield_kick, int nfield_drift, double a_kick,
                           double a_drift, double dtau_kick, double dtau_drift);
@@ -397,6 +399,7 @@ int gev_adj_source_T00(gev_ctx *ctx, const void *phi, const void *T00, const voi
 int gev_adj_source_Tij(gev_ctx *ctx, const void *phi, const void *lS, void *lphi);
 int gev_adj_link_factor(gev_ctx *ctx, const void *phi, const void *L, void *u, void *lphi);
 int gev_adj_project_ft_scalar(gev_ctx *ctx, const void *lchiFT, void *lSijFT);
+int gev_adj_solve_chi(gev_ctx *ctx, const void *lchi, void *lSij, void *chiFT, void *SijFT);
 
 /* ---- background (background.hpp:200-290), Omega_rad/ncdm/fld as given */
 double gev_hconf(double a, double fourpiG, double Omega_m, double Omega_Lambda, double Omega_rad);
