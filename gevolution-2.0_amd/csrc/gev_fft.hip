@@ -407,17 +407,37 @@ __global__ __launch_bounds__(NL * N / 16) void k_r2c_x_multi(Src src, cx<T> *__r
     if constexpr (NC > 2) comp(std::integral_constant<int, 2>{});
     if constexpr (NC > 3) comp(std::integral_constant<int, 3>{});
     if constexpr (NC > 4) comp(std::integral_constant<int, 4>{});
-    if constexpr (NC > 5) comp(std::integral_constant<int, 5>{});
 }
 
-// the six Sij components (Tij at Tij + C M)
-template <typename T, int N> struct SrcSij6 {
+// projectFTscalar takes only the trace-free part of Sij, so two differences of
+// the diagonal and the three off-diagonal components carry it:
+//   0: S_xx - S_zz, 1: S_yy - S_zz, 2: S_xy, 3: S_xz, 4: S_yz
+// (five half spectra to write, transform and read instead of six).
+// From prepareFTsource(phi, Tij, coeff), Tij's component c at Tij + c M:
+template <typename T, int N> struct SrcSij5 {
     const T *phi, *Tij;
     int64_t M;
     T coeff;
     template <int C> __device__ __forceinline__ cx<T> get(int64_t L, int n) const
     {
-        return SrcSij<T, N, C>{phi, Tij + C * M, coeff}(L, n);
+        auto S = [&](auto cc) {
+            constexpr int K = decltype(cc)::value;
+            return SrcSij<T, N, K>{phi, Tij + K * M, coeff}(L, n);
+        };
+        if constexpr (C < 2)
+            return S(std::integral_constant<int, C == 0 ? 0 : 3>{}) - S(std::integral_constant<int, 5>{});
+        else return S(std::integral_constant<int, C == 2 ? 1 : C == 3 ? 2 : 4>{});
+    }
+};
+// and from Sij itself
+template <typename T, int N> struct SrcTraceless {
+    const T *Sij;
+    int64_t M;
+    template <int C> __device__ __forceinline__ cx<T> get(int64_t L, int n) const
+    {
+        auto S = [&](int c) { return SrcPlain<T, N>{Sij + c * M}(L, n); };
+        if constexpr (C < 2) return S(C == 0 ? 0 : 3) - S(5);
+        else return S(C == 2 ? 1 : C == 3 ? 2 : 4);
     }
 };
 
@@ -658,12 +678,14 @@ struct ZParams {
 };
 
 // ============================ y pass of Sij forming the groups of the z solve ==
-// The y transforms of the six Sij components (x-transformed, in place at
-// data + c NK) of TX adjacent kx columns and one z, each output mode added
-// with its (kx, ky) weight of projectFTscalar into the three groups that the
-// z solve transforms (gevolution.hpp:317-323 with g = gridk2, k = kshift):
+// The y transforms of the five trace-free Sij combinations (SrcSij5,
+// x-transformed, at data + c NK) of TX adjacent kx columns and one z, each
+// output mode added with its (kx, ky) weight of projectFTscalar into the three
+// groups that the z solve transforms (gevolution.hpp:317-323 with g = gridk2,
+// k = kshift; U = S_xx - S_zz, V = S_yy - S_zz):
 //   A = (g1 - 2 g0) S_xx - 6 k0 k1 S_xy + (g0 - 2 g1) S_yy + (g0 + g1) S_zz
-//   B = S_xx + S_yy - 2 S_zz,   C = -6 (k0 S_xz + k1 S_yz)
+//     = (g1 - 2 g0) U + (g0 - 2 g1) V - 6 k0 k1 S_xy
+//   B = S_xx + S_yy - 2 S_zz = U + V,   C = -6 (k0 S_xz + k1 S_yz)
 // written over components 0..2 (every column of the workgroup is read before
 // any is written; no other workgroup touches them).  Padding columns
 // (kx > N/2) get 0.  Replaces six y passes and the z solve's reads of six
@@ -723,17 +745,14 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int
                 A[s] = v[s] * (gkl[row] - (T)2 * g0);
                 B[s] = v[s];
             } else if constexpr (c == 1) {
-                A[s] = A[s] + (k0m * ksl[row]) * v[s];
-            } else if constexpr (c == 2) {
-                C[s] = k0m * v[s];
-            } else if constexpr (c == 3) {
                 A[s] = A[s] + v[s] * (g0 - (T)2 * gkl[row]);
                 B[s] = B[s] + v[s];
-            } else if constexpr (c == 4) {
-                C[s] = C[s] + (ksl[row] * (T)-6) * v[s];
+            } else if constexpr (c == 2) {
+                A[s] = A[s] + (k0m * ksl[row]) * v[s];
+            } else if constexpr (c == 3) {
+                C[s] = k0m * v[s];
             } else {
-                A[s] = A[s] + v[s] * (g0 + gkl[row]);
-                B[s] = B[s] - v[s] * (T)2;
+                C[s] = C[s] + (ksl[row] * (T)-6) * v[s];
             }
         }
     };
@@ -742,7 +761,6 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int
     comp(std::integral_constant<int, 2>{});
     comp(std::integral_constant<int, 3>{});
     comp(std::integral_constant<int, 4>{});
-    comp(std::integral_constant<int, 5>{});
     // (selects on the scalar parts: a select of whole structs becomes a select
     // of their addresses, which keeps the arrays out of registers)
     auto put = [&](cx<T> *dst, int s, cx<T> val) {
@@ -1046,8 +1064,7 @@ static void zsolve_chain(gev_ctx *c, int op, const T *rin, int nin, cx<T> *ftin,
     if (op == ZOP_SCALAR && !plane_size<T>(N)) {
         // x passes, then the y pass that forms the three groups of projectFTscalar
         if constexpr (!plane_size<T>(N)) {
-            for (int i = 0; i < nin; i++)
-                launch_r2c<T, N>(rin + i * c->M, ftin + i * c->NK, c->P, (int64_t)N * N, tw, c->stream);
+            launch_r2c_multi<T, N, 5>(SrcTraceless<T, N>{rin, c->M}, ftin, c->P, c->NK, (int64_t)N * N, tw, c->stream);
             launch_col_comb<T, N>(ftin, c->P, c->NK, tw, zp, c->stream);
             launch_zsolve<T, N, ZOP_SCALAR3>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
         }
@@ -1203,7 +1220,7 @@ static void chi_from_Tij_chain(gev_ctx *c, const T *phi, T *Tij, T coeff, cx<T> 
         launch_fwd_plane<T, N>(c, CompSij<T, N>{phi, Tij, c->M, coeff}, SijFT, 6, tw);
         launch_zsolve<T, N, ZOP_SCALAR>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
     } else {
-        launch_r2c_multi<T, N, 6>(SrcSij6<T, N>{phi, Tij, c->M, coeff}, SijFT, c->P, c->NK, nl, tw, c->stream);
+        launch_r2c_multi<T, N, 5>(SrcSij5<T, N>{phi, Tij, c->M, coeff}, SijFT, c->P, c->NK, nl, tw, c->stream);
         launch_col_comb<T, N>(SijFT, c->P, c->NK, tw, zp, c->stream);
         launch_zsolve<T, N, ZOP_SCALAR3>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
     }
