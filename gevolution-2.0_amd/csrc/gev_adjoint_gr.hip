@@ -21,7 +21,6 @@
 // order follows atomic arbitration).  Per-particle adjoints lx, lq are [3][n]
 // arrays indexed by particle ID, as in the Newtonian adjoint; positions in box
 // units (d/dx = N d/dr).
-#include <array>
 #include <type_traits>
 
 #include "gev_common.hpp"
@@ -371,37 +370,6 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
     }
 }
 
-// One field's sites that the stencils of a tile of cells touch, in LDS: the
-// box of BX x BY x BZ sites from (x0, y0, z0) - (LX, LY, LZ), from entry OFF.
-template <int BX, int BY, int BZ, int LX, int LY, int LZ, int OFF> struct StencilBox {
-    static constexpr int N = BX * BY * BZ, END = OFF + N;
-    __device__ static __forceinline__ uint32_t site_of(int e, int x0, int y0, int z0, int mesh)
-    {
-        const uint32_t msk = (uint32_t)mesh - 1;
-        const int ex = e % BX, ey = (e / BX) % BY, ez = e / (BX * BY);
-        return ((uint32_t)(x0 - LX + ex) & msk) +
-               (uint32_t)mesh * (((uint32_t)(y0 - LY + ey) & msk) + (uint32_t)mesh * ((uint32_t)(z0 - LZ + ez) & msk));
-    }
-    // the box's entry for offset (-LX, -LY, -LZ) of cell (cx, cy, cz) of the tile:
-    // every stencil offset adds a constant >= 0 to it, which the LDS
-    // instructions take as their immediate (cx, cy, cz known to be small and
-    // unsigned)
-    __device__ static __forceinline__ uint32_t corner(uint32_t cx, uint32_t cy, uint32_t cz)
-    {
-        return OFF + cx + BX * (cy + BY * cz);
-    }
-    __device__ static __forceinline__ uint32_t step(int dx, int dy, int dz)
-    {
-        return (uint32_t)((dx + LX) + BX * ((dy + LY) + BY * (dz + LZ)));
-    }
-};
-template <typename T, class X> struct BoxField {
-    using Box = X;
-    const T *lds;
-    uint32_t o;  // X::corner of the particle's cell
-    __device__ __forceinline__ T operator()(int dx, int dy, int dz) const { return lds[o + X::step(dx, dy, dz)]; }
-};
-
 // The tiled reverse kick + drift: one workgroup per tile of TX x TY x TZ cells
 // reads the fields its particles' stencils touch from LDS, as the forward
 // update does, and sums the field adjoints in FP64 LDS accumulators over the
@@ -423,11 +391,11 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
                                                           const T *__restrict__ Bi, T *lx, T *lq, T *lphi, T *lchi,
                                                           T *lB, int64_t M, AdjKD s)
 {
-    using XP = StencilBox<TX + 3, TY + 3, TZ + 3, 1, 1, 1, 0>;
-    using XC = StencilBox<TX + 1, TY + 1, TZ + 1, 0, 0, 0, XP::END>;
-    using X0 = StencilBox<TX + 2, TY + 1, TZ + 1, 1, 0, 0, XC::END>;
-    using X1 = StencilBox<TX + 1, TY + 2, TZ + 1, 0, 1, 0, X0::END>;
-    using X2 = StencilBox<TX + 1, TY + 1, TZ + 2, 0, 0, 1, X1::END>;
+    using XP = typename KickBoxes<TX, TY, TZ>::P;
+    using XC = typename KickBoxes<TX, TY, TZ>::C;
+    using X0 = typename KickBoxes<TX, TY, TZ>::B0;
+    using X1 = typename KickBoxes<TX, TY, TZ>::B1;
+    using X2 = typename KickBoxes<TX, TY, TZ>::B2;
     constexpr int NROW = TY * TZ;
     __shared__ T fld[X2::END];
     __shared__ double acc[X2::END];
@@ -436,36 +404,18 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
     int x0, y0, z0;
     tile_origin<TX, TY, TZ>(N, x0, y0, z0);
     const int nfmax = s.nf_k > s.nf_d ? s.nf_k : s.nf_d;
-    // all of a thread's field loads are requested before the first LDS write
-    auto load = [&](auto box, const T *f, bool on) {
-        using X = decltype(box);
-        std::array<T, (X::N + NT - 1) / NT> t;
-#pragma unroll
-        for (int k = 0; k < (int)t.size(); k++) {
-            const int e = tid + k * NT;
-            t[k] = on && e < X::N ? f[X::site_of(e, x0, y0, z0, N)] : (T)0;
-        }
-        return t;
-    };
-    auto put = [&](auto box, const auto &t) {
-        using X = decltype(box);
-#pragma unroll
-        for (int k = 0; k < (int)t.size(); k++) {
-            const int e = tid + k * NT;
-            if (e < X::N) fld[X::END - X::N + e] = t[k];
-        }
-    };
     {
-        const auto tp = load(XP{}, phi, true);
-        const auto tc = load(XC{}, chi, nfmax >= 2);
-        const auto t0 = load(X0{}, Bi, nfmax >= 3);
-        const auto t1 = load(X1{}, Bi + M, nfmax >= 3);
-        const auto t2 = load(X2{}, Bi + 2 * M, nfmax >= 3);
-        put(XP{}, tp);
-        put(XC{}, tc);
-        put(X0{}, t0);
-        put(X1{}, t1);
-        put(X2{}, t2);
+        // all of a thread's field loads are requested before the first LDS write
+        const auto tp = box_load<XP, NT>(phi, true, x0, y0, z0, N);
+        const auto tc = box_load<XC, NT>(chi, nfmax >= 2, x0, y0, z0, N);
+        const auto t0 = box_load<X0, NT>(Bi, nfmax >= 3, x0, y0, z0, N);
+        const auto t1 = box_load<X1, NT>(Bi + M, nfmax >= 3, x0, y0, z0, N);
+        const auto t2 = box_load<X2, NT>(Bi + 2 * M, nfmax >= 3, x0, y0, z0, N);
+        box_put<XP, NT>(fld, tp);
+        box_put<XC, NT>(fld, tc);
+        box_put<X0, NT>(fld, t0);
+        box_put<X1, NT>(fld, t1);
+        box_put<X2, NT>(fld, t2);
     }
     for (int e = tid; e < X2::END; e += NT) acc[e] = 0.0;
     int32_t rb0, incl;

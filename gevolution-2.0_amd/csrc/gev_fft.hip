@@ -407,14 +407,20 @@ __global__ __launch_bounds__(NL * N / 16) void k_r2c_x_multi(Src src, cx<T> *__r
     if constexpr (NC > 2) comp(std::integral_constant<int, 2>{});
     if constexpr (NC > 3) comp(std::integral_constant<int, 3>{});
     if constexpr (NC > 4) comp(std::integral_constant<int, 4>{});
+    if constexpr (NC > 5) comp(std::integral_constant<int, 5>{});
 }
 
 // projectFTscalar takes only the trace-free part of Sij, so two differences of
 // the diagonal and the three off-diagonal components carry it:
 //   0: S_xx - S_zz, 1: S_yy - S_zz, 2: S_xy, 3: S_xz, 4: S_yz
-// (five half spectra to write, transform and read instead of six).
+// (five half spectra to write, transform and read instead of six: 512^3 FP64
+// phi + chi + B solves 20.48 -> 19.82 ms).  FP64 only: in FP32 the six
+// components as they are gain less (1 % of a 512^3 cycle) than what keeping
+// the mixed form's chi unchanged to the last bit is worth, since particles at
+// a cell face move their link deposits by a whole site on a last-bit change.
+template <typename T> constexpr int sij_spectra() { return sizeof(T) == 8 ? 5 : 6; }
 // From prepareFTsource(phi, Tij, coeff), Tij's component c at Tij + c M:
-template <typename T, int N> struct SrcSij5 {
+template <typename T, int N> struct SrcSijX {
     const T *phi, *Tij;
     int64_t M;
     T coeff;
@@ -424,19 +430,21 @@ template <typename T, int N> struct SrcSij5 {
             constexpr int K = decltype(cc)::value;
             return SrcSij<T, N, K>{phi, Tij + K * M, coeff}(L, n);
         };
-        if constexpr (C < 2)
+        if constexpr (sij_spectra<T>() == 6) return S(std::integral_constant<int, C>{});
+        else if constexpr (C < 2)
             return S(std::integral_constant<int, C == 0 ? 0 : 3>{}) - S(std::integral_constant<int, 5>{});
         else return S(std::integral_constant<int, C == 2 ? 1 : C == 3 ? 2 : 4>{});
     }
 };
 // and from Sij itself
-template <typename T, int N> struct SrcTraceless {
+template <typename T, int N> struct SrcPlainX {
     const T *Sij;
     int64_t M;
     template <int C> __device__ __forceinline__ cx<T> get(int64_t L, int n) const
     {
         auto S = [&](int c) { return SrcPlain<T, N>{Sij + c * M}(L, n); };
-        if constexpr (C < 2) return S(C == 0 ? 0 : 3) - S(5);
+        if constexpr (sij_spectra<T>() == 6) return S(C);
+        else if constexpr (C < 2) return S(C == 0 ? 0 : 3) - S(5);
         else return S(C == 2 ? 1 : C == 3 ? 2 : 4);
     }
 };
@@ -678,8 +686,9 @@ struct ZParams {
 };
 
 // ============================ y pass of Sij forming the groups of the z solve ==
-// The y transforms of the five trace-free Sij combinations (SrcSij5,
-// x-transformed, at data + c NK) of TX adjacent kx columns and one z, each
+// The y transforms of the six Sij components, or in FP64 the five trace-free
+// combinations of SrcSijX (x-transformed, at data + c NK), of TX adjacent kx
+// columns and one z, each
 // output mode added with its (kx, ky) weight of projectFTscalar into the three
 // groups that the z solve transforms (gevolution.hpp:317-323 with g = gridk2,
 // k = kshift; U = S_xx - S_zz, V = S_yy - S_zz):
@@ -694,6 +703,7 @@ template <typename T, int L, int TX>
 __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int64_t NK, const cx<T> *__restrict__ tw,
                                                          const double *__restrict__ gk2, const cx<double> *__restrict__ ks)
 {
+    constexpr int NIN = sij_spectra<T>();
     constexpr int NT = TX * L / 8;
     __shared__ cx<T> lds[TX * (L + 1)];
     __shared__ cx<T> twl[L];
@@ -741,7 +751,24 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int
 #pragma unroll
         for (int s = 0; s < 8; s++) {
             const int row = rows[s];
-            if constexpr (c == 0) {
+            if constexpr (NIN == 6) {
+                if constexpr (c == 0) {
+                    A[s] = v[s] * (gkl[row] - (T)2 * g0);
+                    B[s] = v[s];
+                } else if constexpr (c == 1) {
+                    A[s] = A[s] + (k0m * ksl[row]) * v[s];
+                } else if constexpr (c == 2) {
+                    C[s] = k0m * v[s];
+                } else if constexpr (c == 3) {
+                    A[s] = A[s] + v[s] * (g0 - (T)2 * gkl[row]);
+                    B[s] = B[s] + v[s];
+                } else if constexpr (c == 4) {
+                    C[s] = C[s] + (ksl[row] * (T)-6) * v[s];
+                } else {
+                    A[s] = A[s] + v[s] * (g0 + gkl[row]);
+                    B[s] = B[s] - v[s] * (T)2;
+                }
+            } else if constexpr (c == 0) {
                 A[s] = v[s] * (gkl[row] - (T)2 * g0);
                 B[s] = v[s];
             } else if constexpr (c == 1) {
@@ -761,6 +788,7 @@ __global__ __launch_bounds__(TX * L / 8) void k_col_comb(cx<T> *data, int P, int
     comp(std::integral_constant<int, 2>{});
     comp(std::integral_constant<int, 3>{});
     comp(std::integral_constant<int, 4>{});
+    if constexpr (NIN == 6) comp(std::integral_constant<int, 5>{});
     // (selects on the scalar parts: a select of whole structs becomes a select
     // of their addresses, which keeps the arrays out of registers)
     auto put = [&](cx<T> *dst, int s, cx<T> val) {
@@ -1064,7 +1092,7 @@ static void zsolve_chain(gev_ctx *c, int op, const T *rin, int nin, cx<T> *ftin,
     if (op == ZOP_SCALAR && !plane_size<T>(N)) {
         // x passes, then the y pass that forms the three groups of projectFTscalar
         if constexpr (!plane_size<T>(N)) {
-            launch_r2c_multi<T, N, 5>(SrcTraceless<T, N>{rin, c->M}, ftin, c->P, c->NK, (int64_t)N * N, tw, c->stream);
+            launch_r2c_multi<T, N, sij_spectra<T>()>(SrcPlainX<T, N>{rin, c->M}, ftin, c->P, c->NK, (int64_t)N * N, tw, c->stream);
             launch_col_comb<T, N>(ftin, c->P, c->NK, tw, zp, c->stream);
             launch_zsolve<T, N, ZOP_SCALAR3>(ftin, ftout, c->P, c->NK, tw, zp, c->stream);
         }
@@ -1220,7 +1248,7 @@ static void chi_from_Tij_chain(gev_ctx *c, const T *phi, T *Tij, T coeff, cx<T> 
         launch_fwd_plane<T, N>(c, CompSij<T, N>{phi, Tij, c->M, coeff}, SijFT, 6, tw);
         launch_zsolve<T, N, ZOP_SCALAR>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
     } else {
-        launch_r2c_multi<T, N, 5>(SrcSij5<T, N>{phi, Tij, c->M, coeff}, SijFT, c->P, c->NK, nl, tw, c->stream);
+        launch_r2c_multi<T, N, sij_spectra<T>()>(SrcSijX<T, N>{phi, Tij, c->M, coeff}, SijFT, c->P, c->NK, nl, tw, c->stream);
         launch_col_comb<T, N>(SijFT, c->P, c->NK, tw, zp, c->stream);
         launch_zsolve<T, N, ZOP_SCALAR3>(SijFT, chiFT, c->P, c->NK, tw, zp, c->stream);
     }

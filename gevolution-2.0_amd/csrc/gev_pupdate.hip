@@ -45,12 +45,13 @@ template <typename T> __device__ __forceinline__ void idle_pos(int x0, int y0, i
 }
 
 // One particle of a kick / drift pass: the stencil values come from the
-// staged box fields[f * FS + ...] of a tile with origin (x0, y0, z0) and box
-// pitch SX, SY.  Writes q, position and cell; returns the new cell.
-template <typename T, int F, int SX, int SY>
+// tile's staged boxes (KickBoxes).  Writes q, position and cell; returns the
+// new cell.
+template <typename T, int F, int TX, int TY, int TZ>
 __device__ __forceinline__ int32_t upd_particle(const PV<T> &v, const UpdParams &u, int64_t p, int32_t cc, T xk[3],
-                                                T q[3], const T *fields, int x0, int y0, int z0, int FS, double &ret)
+                                                T q[3], const T *fld, double &ret)
 {
+    using BX = KickBoxes<TX, TY, TZ>;
     constexpr bool kick = F & (UPD_KICK_GR | UPD_KICK_NEWTON);
     constexpr bool drift = F & (UPD_DRIFT_GR | UPD_DRIFT_NEWTON);
     const int N = v.N;
@@ -59,12 +60,15 @@ __device__ __forceinline__ int32_t upd_particle(const PV<T> &v, const UpdParams 
     const T Nn = (T)N;
     int32_t newc = 0;
     const int x = cc & (N - 1), y = (cc >> v.lg) & (N - 1), z = cc >> (2 * v.lg);
-    const int o = (x - x0 + 1) + SX * ((y - y0 + 1) + SY * (z - z0 + 1));
+    // the cell inside its tile (tile origins are multiples of the tile's edges)
+    const uint32_t cx = x & (TX - 1), cy = y & (TY - 1), cz = z & (TZ - 1);
     T r[3];
     cell_rel(xk, x, y, z, N, r);
-    FieldLds<T> Fp{fields, o, SX, SX * SY}, Fc{fields + FS, o, SX, SX * SY};
-    FieldLds<T> B0{fields + 2 * FS, o, SX, SX * SY}, B1{fields + 3 * FS, o, SX, SX * SY},
-        B2{fields + 4 * FS, o, SX, SX * SY};
+    const BoxField<T, typename BX::P> Fp{fld, BX::P::corner(cx, cy, cz)};
+    const BoxField<T, typename BX::C> Fc{fld, BX::C::corner(cx, cy, cz)};
+    const BoxField<T, typename BX::B0> B0{fld, BX::B0::corner(cx, cy, cz)};
+    const BoxField<T, typename BX::B1> B1{fld, BX::B1::corner(cx, cy, cz)};
+    const BoxField<T, typename BX::B2> B2{fld, BX::B2::corner(cx, cy, cz)};
     // FP32: kick and drift share weights and stencil reads; FP64 keeps
     // them apart (the shared form needs more registers than it saves)
     if constexpr ((F & (UPD_KICK_GR | UPD_DRIFT_GR)) == (UPD_KICK_GR | UPD_DRIFT_GR) && sizeof(T) == 4) {
@@ -99,18 +103,21 @@ __device__ __forceinline__ int32_t upd_particle(const PV<T> &v, const UpdParams 
 }
 
 template <typename T, int TX, int TY, int TZ, int F, int NT = UpdShape<T>::NT>
-__global__ __launch_bounds__(NT) void k_update_tiled(PV<T> v, UpdParams u, const T *__restrict__ phi,
+__global__ __launch_bounds__(NT, (F == (UPD_KICK_GR | UPD_DRIFT_GR) ? (sizeof(T) == 4 ? 4 : 3) : 1)) void k_update_tiled(PV<T> v, UpdParams u, const T *__restrict__ phi,
                                                         const T *__restrict__ chi, const T *__restrict__ B0g,
                                                         const T *__restrict__ B1g, const T *__restrict__ B2g,
                                                         unsigned long long *maxslot, int32_t *count, int32_t *rank,
                                                         uint32_t *__restrict__ qb)
 {
-    constexpr int SX = TX + 3, SY = TY + 3, SZ = TZ + 3, NS = SX * SY * SZ, NROW = TY * TZ;
-    static_assert(NROW <= 64 && SX <= 64 && (NROW & (NROW - 1)) == 0, "tile shape unsupported by the wave-level staging");
-    __shared__ T fld[5][NS];
+    constexpr int NROW = TY * TZ;
+    static_assert(NROW <= 64 && (NROW & (NROW - 1)) == 0, "one row of the tile per lane");
+    using BX = KickBoxes<TX, TY, TZ>;
+    // the fields a form can read: phi, chi, and B in the GR ones
+    constexpr bool FLD = F != UPD_DRIFT_NEWTON, FLDB = F & (UPD_KICK_GR | UPD_DRIFT_GR);
+    __shared__ T fld[FLDB ? BX::B2::END : (FLD ? BX::C::END : 1)];
     const int N = v.N;
     const uint32_t msk = (uint32_t)N - 1;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
     int x0, y0, z0;
     tile_origin<TX, TY, TZ>(N, x0, y0, z0);
     const int32_t cell0 = (int32_t)((uint32_t)x0 + (uint32_t)N * ((uint32_t)y0 + (uint32_t)N * (uint32_t)z0));
@@ -123,27 +130,16 @@ __global__ __launch_bounds__(NT) void k_update_tiled(PV<T> v, UpdParams u, const
     const int nf_d = (F & UPD_DRIFT_GR) ? u.nf_d : 0;
     const int nfmax = kick ? (nf_k > nf_d ? nf_k : nf_d) : nf_d;
     const bool use_phi = kick || nf_d >= 1, use_chi = nfmax >= 2, use_B = nfmax >= 3;
-    // stage [x0-1, x0+TX+1] x ... : each wave covers RPW box rows per pass, lane -> (row, x)
-    {
-        constexpr int RPW = 64 / SX, NR = SY * SZ, NW = NT / 64;
-        const int sub = lane / SX, lx = lane - sub * SX;
-        const uint32_t gx = (uint32_t)(x0 - 1 + lx) & msk;
-        if (sub < RPW) {
-            for (int row = wv * RPW + sub; row < NR; row += NW * RPW) {
-                const int ly = row % SY, lz = row / SY;
-                const uint32_t g = gx + (uint32_t)N * (((uint32_t)(y0 - 1 + ly) & msk) +
-                                                       (uint32_t)N * ((uint32_t)(z0 - 1 + lz) & msk));
-                const int e = lx + SX * row;
-                if (use_phi) fld[0][e] = phi[g];
-                if (use_chi) fld[1][e] = chi[g];
-                if (use_B) {
-                    fld[2][e] = B0g[g];
-                    fld[3][e] = B1g[g];
-                    fld[4][e] = B2g[g];
-                }
-            }
-        }
-    }
+    // the row starts, then every field value of the tile's boxes: requested
+    // here, stored to LDS after the first particles are requested too, so one
+    // memory round trip covers all of them
+    int32_t rb0, incl;
+    tile_rows_load<TX, TY, NROW>(v.start, N, x0, y0, z0, lane, rb0, incl);
+    const auto tp = box_load<typename BX::P, NT>(phi, use_phi, x0, y0, z0, N);
+    const auto tc = box_load<typename BX::C, NT>(chi, use_chi, x0, y0, z0, N);
+    const auto t0 = box_load<typename BX::B0, NT>(B0g, FLDB && use_B, x0, y0, z0, N);
+    const auto t1 = box_load<typename BX::B1, NT>(B1g, FLDB && use_B, x0, y0, z0, N);
+    const auto t2 = box_load<typename BX::B2, NT>(B2g, FLDB && use_B, x0, y0, z0, N);
     // qb (FP32 form, N >= 16): the largest |q|^2 of the updated particles per
     // block of 8^3 cells (gev_pcls::qbound), for the fixed-point deposits.
     // The blocks of cells [x0-1, x0+TX] x ... (where every particle lands
@@ -159,8 +155,6 @@ __global__ __launch_bounds__(NT) void k_update_tiled(PV<T> v, UpdParams u, const
         for (int e = tid; e < QWN; e += NT) qwin[e] = 0u;
     // particle ranges of the tile's TY*TZ rows, computed by every wave for
     // itself (no barrier before the first particle loads)
-    int32_t rb0, incl;
-    tile_rows_load<TX, TY, NROW>(v.start, N, x0, y0, z0, lane, rb0, incl);
     incl = wave_row_scan(incl, lane);
     const int total = __shfl(incl, NROW - 1, 64);
     const int niter = (total + NT - 1) / NT;  // the same for every lane of the workgroup
@@ -178,6 +172,15 @@ __global__ __launch_bounds__(NT) void k_update_tiled(PV<T> v, UpdParams u, const
         qn[0] = v.q0[lp]; qn[1] = v.q1[lp]; qn[2] = v.q2[lp];
     };
     fetch();
+    if constexpr (FLD) {
+        box_put<typename BX::P, NT>(fld, tp);
+        box_put<typename BX::C, NT>(fld, tc);
+    }
+    if constexpr (FLDB) {
+        box_put<typename BX::B0, NT>(fld, t0);
+        box_put<typename BX::B1, NT>(fld, t1);
+        box_put<typename BX::B2, NT>(fld, t2);
+    }
     __syncthreads();  // staged fields
     double ret = 0.0;
     RankPending rpend{0, 0};
@@ -200,7 +203,7 @@ __global__ __launch_bounds__(NT) void k_update_tiled(PV<T> v, UpdParams u, const
         // maximum over real particles only (a select, no branch)
         double rit = 0.0;
         const int32_t newc =
-            upd_particle<T, F, SX, SY>(v, u, active ? p : v.sink, cc, xk, q, fld[0], x0, y0, z0, NS, rit);
+            upd_particle<T, F, TX, TY, TZ>(v, u, active ? p : v.sink, cc, xk, q, fld, rit);
         ret = active ? fmax(ret, rit) : ret;
         if (qbon && active) {
             const int32_t cq = drift ? newc : cc;
