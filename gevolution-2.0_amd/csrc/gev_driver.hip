@@ -198,12 +198,11 @@ int gev_step(gev_pcls *p, const gev_fields *f, gev_step_state *st)
         RC(mark(c, GEV_PHASE_KICK_DRIFT));
         RC(gev_pcls_rebin_counted(p));
         RC(mark(c, GEV_PHASE_REBIN));
-        RC(gev::read_max_slot(c, &maxv2));  // the scatter leaves the kick's maximum alone
-        if (t00_sums_pending) {
-            double sums[2];
-            RC(gev_ctx_sums(c, sums));  // nothing since the phi solve reduced into these slots
-            st->T00hom = sums[0] / (double)M;
-        }
+        // the kick's maximum (the re-binning leaves it alone) and, in the same
+        // copy, the phi solve's sums, which nothing has reduced into since
+        double src_sum = 0.0;
+        RC(gev::read_max_slot(c, &maxv2, &src_sum));
+        if (t00_sums_pending) st->T00hom = src_sum / (double)M;
         a = gev_rk4bg(a_d, fpg, om, ol, orad, 0.5 * dtau);
         double mv = sqrt(maxv2);
         st->maxvel = mv / sqrt(mv * mv + 1.0); // main.cu:1279-1283

@@ -56,8 +56,9 @@ template <typename T> int prepare_Tij_impl(gev_ctx *ctx, const T *phi, const T *
 template <typename T> int field_sum_impl(gev_ctx *ctx, const T *f, int64_t count, double *sum);
 template <typename T> int field_fill_impl(gev_ctx *ctx, T *f, int64_t count, T v);
 
-// copy the last kick's maximum (FP64 slot) to the host; synchronises the stream
-int read_max_slot(gev_ctx *c, double *out);
+// copy the last kick's maximum (FP64 slot), and with sum0 the first reduction
+// slot, to the host; synchronises the stream
+int read_max_slot(gev_ctx *c, double *out, double *sum0 = nullptr);
 template <typename T>
 int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi, T *lx, T *lq, T *lphi, T *lchi,
                            T *lB, int nf_k, int nf_d, double a_k, double a_d, double dtau_k, double dtau_d);

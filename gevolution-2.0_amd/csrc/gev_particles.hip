@@ -181,11 +181,23 @@ __global__ __launch_bounds__(1024) void k_scan_mid(int32_t *bsum, int64_t nb)
 }
 
 // writes the exclusive prefix of cnt to start and clears cnt for the next count;
-// start[M] = total, or the sum of all counts when total < 0
+// start[M] = total, or the sum of all counts when total < 0.  bsum holds the
+// exclusive prefix of the chunks' sums, or with OWN the sums themselves, which
+// every workgroup then adds up to its own chunk (one launch fewer: up to
+// SCAN_OWN chunks; a 128^3 mesh has 1024)
+template <bool OWN>
 __global__ __launch_bounds__(SCAN_NT) void k_scan_apply(int32_t *__restrict__ cnt, int64_t M,
                                                         const int32_t *__restrict__ bsum, int32_t *__restrict__ start,
                                                         int32_t total)
 {
+    int32_t before = 0;
+    if constexpr (OWN) {
+        int32_t s = 0;
+        for (unsigned j = threadIdx.x; j < blockIdx.x; j += SCAN_NT) s += bsum[j];
+        block_excl_scan(s, before);
+    } else {
+        before = bsum[blockIdx.x];
+    }
     static_assert(SCAN_PER == 8, "two 16-byte vectors per thread");
     // each thread owns SCAN_PER consecutive cells: 16-byte loads and stores
     // where the whole run is inside [0, M) (always when M is a multiple of 8)
@@ -210,7 +222,7 @@ __global__ __launch_bounds__(SCAN_NT) void k_scan_apply(int32_t *__restrict__ cn
 #pragma unroll
     for (int j = 0; j < SCAN_PER; j++) s += v[j];
     int32_t tot;
-    int32_t off = block_excl_scan(s, tot) + bsum[blockIdx.x];
+    int32_t off = block_excl_scan(s, tot) + before;
     int32_t o[SCAN_PER];
 #pragma unroll
     for (int j = 0; j < SCAN_PER; j++) {
@@ -232,6 +244,61 @@ __global__ __launch_bounds__(SCAN_NT) void k_scan_apply(int32_t *__restrict__ cn
         for (int j = 0; j < SCAN_PER; j++)
             if (base + j == M - 1) start[M] = o[j] + v[j];
     }
+}
+
+// The whole scan in one workgroup for up to four cells per thread (a 16^3
+// mesh), whose three small kernels are all launch.  (For 32^3 one workgroup's
+// 32 cells per thread measured slower than two launches.)
+constexpr int SCAN_ONE_NT = 1024;
+constexpr int64_t SCAN_ONE = 4 * SCAN_ONE_NT, SCAN_OWN = 1024;
+__global__ __launch_bounds__(SCAN_ONE_NT) void k_scan_one(int32_t *__restrict__ cnt, int M, int32_t *__restrict__ start)
+{
+    __shared__ int32_t wsum[SCAN_ONE_NT / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, b0 = threadIdx.x * 4;
+    int32_t v[4], s = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[j] = b0 + j < M ? cnt[b0 + j] : 0;
+        s += v[j];
+    }
+    int32_t x = s;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t y = __shfl_up(x, o, 64);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) wsum[w] = x;
+    __syncthreads();
+    int32_t off = x - s;
+    for (int j = 0; j < w; j++) off += wsum[j];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (b0 + j < M) {
+            start[b0 + j] = off;
+            cnt[b0 + j] = 0;
+            off += v[j];
+            if (b0 + j == M - 1) start[M] = off;
+        }
+}
+
+// start = exclusive prefix of cnt (length M), start[M] = total (the sum when
+// total < 0); clears cnt
+static void launch_scan(gev_ctx *ctx, int32_t *cnt, int64_t M, int32_t *start, int32_t total)
+{
+    hipStream_t s = ctx->stream;
+    if (M <= SCAN_ONE) {
+        hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(SCAN_ONE_NT), 0, s, cnt, (int)M, start);
+        return;
+    }
+    const int64_t nb = (M + SCAN_CHUNK - 1) / SCAN_CHUNK;
+    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_NT), 0, s, cnt, M, ctx->scan_blocks);
+    if (nb <= SCAN_OWN) {
+        hipLaunchKernelGGL((k_scan_apply<true>), dim3((unsigned)nb), dim3(SCAN_NT), 0, s, cnt, M, ctx->scan_blocks,
+                           start, total);
+        return;
+    }
+    hipLaunchKernelGGL(k_scan_mid, dim3(1), dim3(1024), 0, s, ctx->scan_blocks, nb);
+    hipLaunchKernelGGL((k_scan_apply<false>), dim3((unsigned)nb), dim3(SCAN_NT), 0, s, cnt, M, ctx->scan_blocks, start,
+                       total);
 }
 
 // Re-binning in two passes: k_perm scatters only the old slot and the cell
@@ -262,6 +329,23 @@ __global__ __launch_bounds__(PT_NT) void k_gather(PV<T> s, PV<T> d, const int32_
     d.q0[j] = s.q0[i]; d.q1[j] = s.q1[i]; d.q2[j] = s.q2[i];
     d.id[j] = s.id[i];
 }
+
+// Both passes in one below PERM_MIN particles, where the second launch costs
+// more than the partial lines (kick + drift calls at 64^3: 137 against 153 us in
+// FP32, 123 against 145 in FP64; equal at 128^3; 512^3 4.07 against 2.63 ms for
+// the pair)
+template <typename T>
+__global__ __launch_bounds__(PT_NT) void k_scatter(PV<T> s, PV<T> d, const int32_t *__restrict__ rank)
+{
+    const int64_t i = (int64_t)blockIdx.x * PT_NT + threadIdx.x;
+    if (i >= s.n) return;
+    const int32_t c = s.cell[i], j = s.start[c] + rank[i];
+    d.p0[j] = s.p0[i]; d.p1[j] = s.p1[i]; d.p2[j] = s.p2[i];
+    d.q0[j] = s.q0[i]; d.q1[j] = s.q1[i]; d.q2[j] = s.q2[i];
+    d.id[j] = s.id[i];
+    d.cell[j] = c;
+}
+constexpr int64_t PERM_MIN = 1 << 20;
 
 // displace_pcls_ic_basic, ic_basic.hpp:65-96 (one field)
 template <typename T>
@@ -337,11 +421,7 @@ template <typename T> int pcls_sort_counted_impl(gev_pcls *p)
     gev_ctx *ctx = p->ctx;
     hipStream_t s = ctx->stream;
     const int64_t M = ctx->M, n = p->n;
-    int64_t nb = (M + SCAN_CHUNK - 1) / SCAN_CHUNK;
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_NT), 0, s, p->cell_count, M, ctx->scan_blocks);
-    hipLaunchKernelGGL(k_scan_mid, dim3(1), dim3(1024), 0, s, ctx->scan_blocks, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_NT), 0, s, p->cell_count, M, ctx->scan_blocks,
-                       p->cell_start, (int32_t)n);
+    launch_scan(ctx, p->cell_count, M, p->cell_start, (int32_t)n);
     p->counts_zero = true;
     if (n > 0) {
         PV<T> src = make_pv<T>(p);
@@ -350,9 +430,13 @@ template <typename T> int pcls_sort_counted_impl(gev_pcls *p)
         dst.q0 = (T *)p->q2[0]; dst.q1 = (T *)p->q2[1]; dst.q2 = (T *)p->q2[2];
         dst.id = p->id2;
         dst.cell = p->cell2;
-        hipLaunchKernelGGL(k_perm, dim3(pblocks(n)), dim3(PT_NT), 0, s, p->cell, p->cell_start, p->rank, p->perm,
-                           p->cell2, n);
-        hipLaunchKernelGGL((k_gather<T>), dim3(pblocks(n)), dim3(PT_NT), 0, s, src, dst, p->perm);
+        if (n < PERM_MIN) {
+            hipLaunchKernelGGL((k_scatter<T>), dim3(pblocks(n)), dim3(PT_NT), 0, s, src, dst, p->rank);
+        } else {
+            hipLaunchKernelGGL(k_perm, dim3(pblocks(n)), dim3(PT_NT), 0, s, p->cell, p->cell_start, p->rank, p->perm,
+                               p->cell2, n);
+            hipLaunchKernelGGL((k_gather<T>), dim3(pblocks(n)), dim3(PT_NT), 0, s, src, dst, p->perm);
+        }
         for (int d = 0; d < 3; d++) {
             std::swap(p->pos[d], p->pos2[d]);
             std::swap(p->q[d], p->q2[d]);
@@ -372,11 +456,7 @@ int scan_exclusive_counts(gev_ctx *ctx, int32_t *cnt, int64_t M, int32_t *start)
         gev_set_error("scan_exclusive_counts: length outside the context's scan space");
         return GEV_ERR_ARG;
     }
-    hipStream_t s = ctx->stream;
-    hipLaunchKernelGGL(k_scan_reduce, dim3((unsigned)nb), dim3(SCAN_NT), 0, s, cnt, M, ctx->scan_blocks);
-    hipLaunchKernelGGL(k_scan_mid, dim3(1), dim3(1024), 0, s, ctx->scan_blocks, nb);
-    hipLaunchKernelGGL(k_scan_apply, dim3((unsigned)nb), dim3(SCAN_NT), 0, s, cnt, M, ctx->scan_blocks, start,
-                       (int32_t)-1);
+    launch_scan(ctx, cnt, M, start, -1);
     GEV_HIP(hipGetLastError());
     return GEV_OK;
 }

@@ -323,11 +323,13 @@ template <typename T> static int launch_update(gev_pcls *p, const UpdParams &u, 
     return GEV_OK;
 }
 
-int read_max_slot(gev_ctx *c, double *out)
+int read_max_slot(gev_ctx *c, double *out, double *sum0)
 {
-    GEV_HIP(hipMemcpyAsync(c->red_host, c->red + 8, sizeof(double), hipMemcpyDeviceToHost, c->stream));
+    const int first = sum0 ? 0 : 8;
+    GEV_HIP(hipMemcpyAsync(c->red_host, c->red + first, (9 - first) * sizeof(double), hipMemcpyDeviceToHost, c->stream));
     GEV_HIP(hipStreamSynchronize(c->stream));
-    *out = c->red_host[0];
+    *out = c->red_host[8 - first];
+    if (sum0) *sum0 = c->red_host[0];
     return GEV_OK;
 }
 
