@@ -60,11 +60,11 @@ __device__ __forceinline__ void lds_add(int32_t *a, float v)
     asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
     __hip_atomic_fetch_add(a, r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-__device__ __forceinline__ void lds_add(uint64_t *a, float v)
+__device__ __forceinline__ void lds_add(int64_t *a, float v)
 {
     int32_t r;
     asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(v));
-    __hip_atomic_fetch_add(a, (uint64_t)(uint32_t)r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __hip_atomic_fetch_add(a, (int64_t)r, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // accumulator of a kind and precision: fixed point for the FP32 form of the
 // physical projections (their values are bounded by the particles' energies);
@@ -72,17 +72,16 @@ __device__ __forceinline__ void lds_add(uint64_t *a, float v)
 template <typename T, int KIND> struct DepAcc { using type = double; };
 template <int KIND> struct DepAcc<float, KIND> { using type = int32_t; };
 template <> struct DepAcc<float, 4> { using type = double; };  // DEP_VEC3
-// The tiles of long rows deposit masses only (no phi box).  Rows of 64 cells
-// add the CIC weights to 64-bit integers at the fixed scale 2^30, which needs
-// no bound on a site's count: one from the runs of a long row would cost up to
-// 2 of the 30 bits, and one from shorter stretches reads the whole cell-start
-// array (1024^3, 0.09 particles per cell: 8.99 against 7.9 ms).  With one
-// particle per cell the 64-bit atomics cost more than that (512^3, 32x8x4:
-// 1.86 against 1.69 ms).  Error of the density against FP64, rms: 256^3 with
-// 0.09 particles per cell 3.2e-8 (16x8x8: 8.9e-8).
+// The tiles of long rows deposit masses only (no phi box), on sparse meshes.
+// They add the CIC weights to 64-bit integers at the fixed scale 2^30, which
+// needs no bound on a site's count: one from the runs of a long row would cost
+// up to 2 of the 30 bits, and one from shorter stretches reads the whole
+// cell-start array (1024^3, 0.09 particles per cell: 8.99 against 7.9 ms).
+// Error of the density against FP64, rms: 256^3 with 0.09 particles per cell
+// 3.2e-8 (16x8x8 in 32 bits: 8.9e-8).
 template <typename T, int KIND, int TX> struct DepRow {
-    static constexpr bool MASS = KIND == DEP_T00 && TX > 16, WIDE = MASS && TX >= 64;
-    using AccT = std::conditional_t<WIDE, uint64_t, typename DepAcc<T, KIND>::type>;
+    static constexpr bool MASS = KIND == DEP_T00 && TX > 16;
+    using AccT = std::conditional_t<MASS, int64_t, typename DepAcc<T, KIND>::type>;
 };
 
 #ifndef DEP_CHUNK_X4
@@ -106,7 +105,7 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
     constexpr int NPH = PX * PY * PZ;
     static_assert(NSEG <= PT_NT, "one run per thread in the scan");
     using AccT = typename DepRow<T, KIND, TX>::AccT;
-    constexpr bool MASS = DepRow<T, KIND, TX>::MASS, WIDE = DepRow<T, KIND, TX>::WIDE;
+    constexpr bool MASS = DepRow<T, KIND, TX>::MASS;
     constexpr bool FIX = sizeof(AccT) == 4;
     constexpr int NW = PT_NT / 64;
     static_assert(!FIX || (TY * TZ <= 64 && NS % 4 == 0 && TX % 4 == 0), "fixed-point tile shape");
@@ -116,10 +115,6 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
     __shared__ int32_t rbeg[NSEG + 1];
     __shared__ int32_t rst[NSEG];
     __shared__ int32_t wsum[PT_NT / 64];
-    // particles per stretch of SX owned cells and the one before it, so that
-    // the bound on a site's count does not grow with TX
-    constexpr int SX = 8, NK = FIX && MASS ? TX / SX : 1;
-    __shared__ int32_t cst[NK > 1 ? NR * NK : 1];
     const int N = v.N;
     const uint32_t msk = (uint32_t)N - 1;
     const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
@@ -194,17 +189,6 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
         rst[t] = s0;
         len = v.start[c1] - s0;
     }
-    if constexpr (NK > 1) {
-        // mostly by the waves without runs
-        static_assert(NR * NK <= PT_NT, "one stretch per thread");
-        const int e = t - (PT_NT - NR * NK);
-        if (e >= 0) {
-            const int k = e % NK, r = e / NK, ly = r % HY, lz = r / HY;
-            const uint32_t row = (uint32_t)N * (((uint32_t)(y0 - 1 + ly) & msk) + (uint32_t)N * ((uint32_t)(z0 - 1 + lz) & msk));
-            const uint32_t c0 = row + (uint32_t)(x0 + SX * k), ch = row + ((uint32_t)(x0 + SX * k - 1) & msk);
-            cst[e] = (v.start[ch + 1] - v.start[ch]) + (v.start[c0 + SX] - v.start[c0]);
-        }
-    }
     int32_t incl = len;
     for (int o = 1; o < 64; o <<= 1) {
         const int32_t y = __shfl_up(incl, o, 64);
@@ -238,18 +222,9 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
         // a site takes the particles of two cells in each of four halo rows,
         // so the four rows' totals bound its particle count (run lengths of the
         // scan; looser than the count of its eight cells by at most the row
-        // length, which costs a few of the 30 bits; rows of more than 16 cells
-        // use the counts of their stretches of SX cells instead)
+        // length, which costs a few of the 30 bits)
         uint32_t cb = 0;
-        if constexpr (NK > 1) {
-            for (int e = lane; e < TY * TZ * NK; e += 64) {
-                const int k = e % NK, sy = (e / NK) % TY, sz = e / (NK * TY);
-                uint32_t c4 = 0;
-#pragma unroll
-                for (int d = 0; d < 4; d++) c4 += (uint32_t)cst[((sy + (d & 1)) + HY * (sz + (d >> 1))) * NK + k];
-                cb = max(cb, c4);
-            }
-        } else if (lane < TY * TZ) {
+        if (lane < TY * TZ) {
             const int sy = lane % TY, sz = lane / TY;
 #pragma unroll
             for (int d = 0; d < 4; d++) {
@@ -435,7 +410,7 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
                     }
                 }
             } else {
-                const T sc = WIDE ? (T)1073741824 : (FIX ? (T)S0 : o);
+                const T sc = MASS ? (T)1073741824 : (FIX ? (T)S0 : o);
 #pragma unroll
                 for (int b = 0; b < 8; b++) {
                     const int bx = (b >> 2) & 1, by = (b >> 1) & 1, bz = b & 1;
@@ -553,8 +528,8 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
     auto grp_of = [&](int c) {
         return KIND == DEP_T00 ? 0 : KIND == DEP_TIJ ? 1 : KIND == DEP_T0I ? 2 : (c == 0 ? 0 : (c < 7 ? 1 : 2));
     };
-    if constexpr (WIDE) fac[0] = mass_d / 1073741824.0;
-    if ((FIX || WIDE) && vec4) {
+    if constexpr (MASS) fac[0] = mass_d / 1073741824.0;
+    if ((FIX || MASS) && vec4) {
         // four consecutive sites of one component per thread and pass: one
         // 16-byte LDS read and one 16-byte store (outputs 16-byte aligned)
         const float ff[3] = {(float)fac[0], (float)fac[1], (float)fac[2]};
@@ -568,7 +543,7 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
             const int g = grp_of(c);
             const float f = g == 0 ? ff[0] : (g == 1 ? ff[1] : ff[2]);
             float4 val;
-            if constexpr (WIDE) {
+            if constexpr (MASS) {
                 const AccT *r = &acc[c][s];
                 val = make_float4((float)r[0] * f, (float)r[1] * f, (float)r[2] * f, (float)r[3] * f);
             } else {
@@ -591,7 +566,7 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
         for (int c = 0; c < C; c++) {
             T *oc = out_of(c);
             const double ms = (T00TIJ && c > 0) ? ((KIND == DEP_T00TIJL && c >= 7) ? mass3_d : mass2_d) : mass_d;
-            T val = FIX || WIDE ? (T)((double)acc[c][s] * fac[grp_of(c)]) : (T)(acc[c][s] * ms);
+            T val = FIX || MASS ? (T)((double)acc[c][s] * fac[grp_of(c)]) : (T)(acc[c][s] * ms);
             if (accumulate) val += oc[gs];
             oc[gs] = val;
         }
@@ -625,20 +600,18 @@ static int dispatch_dep(gev_pcls *p, T *out, const T *phi, double mass, double a
     // Tij keeps 6 (T00+Tij 7) FP64 accumulators per site: the smaller tile holds 4 blocks per CU
     constexpr bool big = KIND != DEP_TIJ && KIND != DEP_T00TIJ && KIND != DEP_T00TIJL;
     if (KIND == DEP_T0I && N >= 32) return launch_dep<T, KIND, 32, 4, 4>(p, out, out2, phi, mass, mass2, a, acc, aux, out3, mass3);
-    // The mass deposit (FP32, no phi box) is mostly set-up and store per tile:
-    // longer rows cut the run lookups per site, as long as a tile holds too few
-    // particles for one workgroup to be the longer wait.  mass + r2c calls at
-    // 16x8x8 and 64x8x4: 1024^3 with 0.09 particles per cell 9.57 and 7.9 ms,
-    // with 0.37 11.2 and 9.5 ms, 512^3 with 0.12 1.19 and 0.94 ms, 256^3 with
-    // 0.12 137 and 128 us; one per cell, 16x8x8, 32x8x4 and 64x8x4 (32-bit):
-    // 512^3 1.80, 1.69, 1.76 ms, 256^3 242, 235, 247 us, 128^3 40.6, 41.7, 45.5 us.
-    // FP64 at 256^3: 388, 386, 450 us.
+    // The mass deposit of a sparse mesh (FP32, no phi box) is mostly set-up and
+    // store per tile: longer rows cut the run lookups per site.  mass + r2c
+    // calls at 16x8x8 and 64x8x4: 1024^3 with 0.09 particles per cell 9.57 and
+    // 7.9 ms, with 0.37 11.2 and 9.5 ms, 512^3 with 0.12 1.19 and 0.94 ms,
+    // 256^3 with 0.12 137 and 128 us.  With one per cell the 64-bit atomics
+    // cost what the rows give (512^3 1.80 and 1.86 ms, 256^3 242 and 252 us at
+    // 32x8x4), and 32-bit sums with a bound as tight as 16x8x8's do too (1.77
+    // ms, 243 us, with crowded cells at 256^3 281 against 274 us).  128^3:
+    // 40.6 against 45.5 us.  FP64 at 256^3: 388 against 450 us.
     if constexpr (KIND == DEP_T00 && sizeof(T) == 4) {
-        if (!phi && N >= 256) {
-            if (2 * p->n < p->ctx->M)
-                return launch_dep<T, KIND, 64, 8, 4>(p, out, out2, phi, mass, mass2, a, acc, aux, out3, mass3);
-            return launch_dep<T, KIND, 32, 8, 4>(p, out, out2, phi, mass, mass2, a, acc, aux, out3, mass3);
-        }
+        if (!phi && N >= 256 && 2 * p->n < p->ctx->M)
+            return launch_dep<T, KIND, 64, 8, 4>(p, out, out2, phi, mass, mass2, a, acc, aux, out3, mass3);
     }
     if (big && N >= 16) return launch_dep<T, KIND, 16, 8, 8>(p, out, out2, phi, mass, mass2, a, acc, aux, out3, mass3);
     if ((KIND == DEP_T00TIJ || KIND == DEP_T00TIJL) && N >= 16)

@@ -1,5 +1,5 @@
 """FP32 mass deposit in long rows (N >= 256: 64 x 8 x 4 cells below one particle
-per two cells, 32 x 8 x 4 from there, 16 x 8 x 8 on smaller meshes), against
+per two cells, 16 x 8 x 8 from there and on smaller meshes), against
 FP64 sums over the same positions.  Offsets are multiples of 2^-16 of a cell,
 held exactly by FP32.  Bound per site, in units of the mass: every addition
 rounds to half a unit of the tile's fixed point, cmax / 2^30, with at most 8 k
