@@ -630,17 +630,37 @@ __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restr
     int x0, y0, z0;
     tile_origin<TX, TY, TZ>(N, x0, y0, z0);
     const bool has_phi = phi != nullptr, has_links = lL != nullptr, out_phi = has_phi && lphi != nullptr;
-    for (int e = tid; e < NS; e += NT) {
-        const int ex = e % SX, ey = (e / SX) % SY, ez = e / (SX * SY);
-        const uint32_t g = ((uint32_t)(x0 + ex) & msk) +
-                           (uint32_t)N * (((uint32_t)(y0 + ey) & msk) + (uint32_t)N * ((uint32_t)(z0 + ez) & msk));
-        fld[0][e] = lT00[g];
+    {
+        // all of a thread's field loads are requested before the first LDS
+        // write, and below a particle's old adjoints with its state, before the
+        // physics instead of after it.  Both reverse kernels: 256^3 mixed 3.86
+        // -> 3.73 ms (IDs in no order 8.25 -> 7.87), 128^3 FP64 754 -> 730 us,
+        // 64^3 mixed 91 -> 84 us (IDs in no order 142 -> 146); the old adjoints
+        // alone 3.76 ms, 757 and 86 us
+        constexpr int NI = (NS + NT - 1) / NT;
+        T ld[NI][11];
 #pragma unroll
-        for (int c = 0; c < 6; c++) fld[1 + c][e] = lTij[c * M + g];
+        for (int k = 0; k < NI; k++) {
+            const int e = min(tid + k * NT, NS - 1);
+            const int ex = e % SX, ey = (e / SX) % SY, ez = e / (SX * SY);
+            const uint32_t g = ((uint32_t)(x0 + ex) & msk) +
+                               (uint32_t)N * (((uint32_t)(y0 + ey) & msk) + (uint32_t)N * ((uint32_t)(z0 + ez) & msk));
+            ld[k][0] = lT00[g];
 #pragma unroll
-        for (int c = 0; c < 3; c++) fld[7 + c][e] = has_links ? lL[c * M + g] : (T)0;
-        fld[10][e] = has_phi ? phi[g] : (T)0;
-        acc[e] = 0.0;
+            for (int c = 0; c < 6; c++) ld[k][1 + c] = lTij[c * M + g];
+#pragma unroll
+            for (int c = 0; c < 3; c++) ld[k][7 + c] = has_links ? lL[c * M + g] : (T)0;
+            ld[k][10] = has_phi ? phi[g] : (T)0;
+        }
+#pragma unroll
+        for (int k = 0; k < NI; k++) {
+            const int e = tid + k * NT;
+            if (e < NS) {
+#pragma unroll
+                for (int c = 0; c < 11; c++) fld[c][e] = ld[k][c];
+                acc[e] = 0.0;
+            }
+        }
     }
     int32_t rb0, incl;
     tile_rows_load<TX, TY, NROW>(v.start, N, x0, y0, z0, lane, rb0, incl);
@@ -658,6 +678,9 @@ __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restr
         T rt[3];
         ref_dist(v, p, x, y, z, rt);
         const T qt[3] = {v.q0[p], v.q1[p], v.q2[p]};
+        T LX[3], LQ[3];
+#pragma unroll
+        for (int j = 0; j < 3; j++) { LX[j] = lx[j * n + id]; LQ[j] = lq[j * n + id]; }
         const int o = (x - x0) + SX * ((y - y0) + SY * (z - z0));
         auto F = [&](int f, int dx, int dy, int dz) -> T { return fld[f][o + dx + SX * dy + SX * SY * dz]; };
         auto sc = [&](int b, T val) {
@@ -668,8 +691,8 @@ __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restr
         adj_gr_deposit_particle<T>(rt, qt, F, has_phi, has_links, N, m00, mij, m0i, a, gx, gq, sc);
 #pragma unroll
         for (int j = 0; j < 3; j++) {
-            lx[j * n + id] += gx[j];
-            lq[j * n + id] += gq[j];
+            lx[j * n + id] = LX[j] + gx[j];
+            lq[j * n + id] = LQ[j] + gq[j];
         }
     }
     if (out_phi) {
