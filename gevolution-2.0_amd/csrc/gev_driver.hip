@@ -155,26 +155,33 @@ int gev_step(gev_pcls *p, const gev_fields *f, gev_step_state *st)
             // scalarFT; both read phi): they run on the side stream while the
             // chi solve runs on the main one, which waits for them before the
             // kick.  Phases: deposit_T0i is the fork (~0), solve_chi the chi
-            // solve beside them, solve_B the wait after it.
+            // solve beside them, solve_B the wait after it.  Up to N = 64 the
+            // fork and join cost more than the overlap gives, and B follows chi
+            // on the main stream (eight GR cycles beside / after: 16^3 FP64
+            // 1024 / 970 us, 32^3 1073 / 1014, 64^3 mixed 1205 / 1172; four at
+            // 128^3 FP64 3336 / 3484, mixed 1995 / 2007).
+            const bool beside = c->N > 64;
+            auto solve_B = [&]() -> int {
+                if (t0i_links) return gev_solve_vector_T0i_links(c, f->Bi, f->phi, f->BiFT, fpg * dx * dx, 0.0);
+                const int rc = gev_project_T0i(p, f->Bi, f->phi, 1.0, 0);
+                return rc ? rc : gev_solve_vector(c, f->Bi, f->BiFT, fpg * dx * dx, 0.0);
+            };
             RC(mark(c, GEV_PHASE_SOURCE_TIJ));
-            GEV_HIP(hipEventRecord(c->fork, c->stream));
-            GEV_HIP(hipStreamWaitEvent(c->side, c->fork, 0));
-            hipStream_t main_stream = c->stream;
-            c->stream = c->side;
-            int rc_side;
-            if (t0i_links) {
-                rc_side = gev_solve_vector_T0i_links(c, f->Bi, f->phi, f->BiFT, fpg * dx * dx, 0.0);
-            } else {
-                rc_side = gev_project_T0i(p, f->Bi, f->phi, 1.0, 0);
-                if (!rc_side) rc_side = gev_solve_vector(c, f->Bi, f->BiFT, fpg * dx * dx, 0.0);
+            if (beside) {
+                GEV_HIP(hipEventRecord(c->fork, c->stream));
+                GEV_HIP(hipStreamWaitEvent(c->side, c->fork, 0));
+                hipStream_t main_stream = c->stream;
+                c->stream = c->side;
+                const int rc_side = solve_B();
+                c->stream = main_stream;
+                GEV_HIP(hipEventRecord(c->join, c->side));
+                RC(rc_side);
             }
-            c->stream = main_stream;
-            GEV_HIP(hipEventRecord(c->join, c->side));
-            RC(rc_side);
             RC(mark(c, GEV_PHASE_DEPOSIT_T0I));
             RC(gev_solve_chi_Tij(c, f->phi, f->Sij, 2. * fpg * dx * dx / a, f->chi, f->SijFT, f->scalarFT));
             RC(mark(c, GEV_PHASE_SOLVE_CHI));
-            GEV_HIP(hipStreamWaitEvent(c->stream, c->join, 0));
+            if (beside) GEV_HIP(hipStreamWaitEvent(c->stream, c->join, 0));
+            else RC(solve_B());
         } else {
             RC(gev_prepare_source_Tij(c, f->phi, f->Sij, f->Sij, 2. * fpg * dx * dx / a));
             RC(mark(c, GEV_PHASE_SOURCE_TIJ));
