@@ -819,6 +819,14 @@ static void launch_col_comb(cx<T> *data, int P, int64_t NK, const cx<T> *tw, con
 // 512^3 B solve; the scalar projection and FP64 measured no better that way
 template <typename T, int L, int OP> constexpr int zs_waves() { return (OP == ZOP_VECTOR && sizeof(T) == 4 && L >= 128) ? 4 : 1; }
 
+// The type of ZOP_SCALAR's weights and group sums.  Up to L = 64 FP64 in both
+// forms, as k_project_ft_scalar's: these meshes are bound by latency and FP64
+// costs no time there (mixed chi solves of 16^3, 32^3, 64^3 14.6, 15.7, 20.9 us
+// with FP32 sums, 14.5, 15.3, 21.0 with FP64 ones), and a Sij that is all trace
+// then gives nothing instead of 1e-8 to 1e-7 of its single components' chi.  At
+// 128 it costs 1 % (56.8, 57.4 us): the transform's precision, as k_col_comb.
+template <typename T, int L> using scalar_weight_t = std::conditional_t<(L <= 64), double, T>;
+
 template <typename T, int L, int TX, int OP>
 __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(const cx<T> *in, cx<T> *out, int P, int64_t NK,
                                                        const cx<T> *__restrict__ tw, ZParams zp)
@@ -1022,22 +1030,26 @@ __global__ __launch_bounds__(TX * L / 8, (zs_waves<T, L, OP>())) void k_zsolve(c
                 forward(kind, st);
             } else {
                 // from the six components, each group formed in the loads of
-                // its transform (the formulas of k_col_comb)
+                // its transform (the formulas of k_col_comb) and rounded once
                 const cx<T> *src = in + off;
                 auto ld = [&](int line, int row) {
                     const int kx = ct * TX + line;
                     const bool valid = kx <= H;  // padding columns give 0 above
                     const cx<T> *e = src + (int64_t)row * stride + line;
-                    const T g0 = valid ? (T)gkd[kx] : (T)0, g1 = (T)gy;
-                    const cx<T> k0 = valid ? mk((T)ksd[kx].x, (T)ksd[kx].y) : mk((T)0, (T)0);
-                    const cx<T> k1 = mk((T)kyv.x, (T)kyv.y);
+                    using W = scalar_weight_t<T, L>;
+                    auto at = [&](int c) { return mk((W)e[c * NK].x, (W)e[c * NK].y); };
+                    const W g0 = valid ? (W)gkd[kx] : (W)0, g1 = (W)gy;
+                    const cx<W> k0 = valid ? mk((W)ksd[kx].x, (W)ksd[kx].y) : mk((W)0, (W)0);
+                    const cx<W> k1 = mk((W)kyv.x, (W)kyv.y);
+                    cx<W> r;
                     if constexpr (K == 0)
-                        return e[0] * (g1 - (T)2 * g0) + ((k0 * (T)-6) * k1) * e[NK] + e[3 * NK] * (g0 - (T)2 * g1) +
-                               e[5 * NK] * (g0 + g1);
+                        r = at(0) * (g1 - (W)2 * g0) + ((k0 * (W)-6) * k1) * at(1) + at(3) * (g0 - (W)2 * g1) +
+                            at(5) * (g0 + g1);
                     else if constexpr (K == 1)
-                        return e[0] + e[3 * NK] - e[5 * NK] * (T)2;
+                        r = at(0) + at(3) - at(5) * (W)2;
                     else
-                        return (k0 * (T)-6) * e[2 * NK] + (k1 * (T)-6) * e[4 * NK];
+                        r = (k0 * (W)-6) * at(2) + (k1 * (W)-6) * at(4);
+                    return mk((T)r.x, (T)r.y);
                 };
                 if constexpr (K == 0) {
                     reg_fft<T, L, TX, true, 1, false, 1>(lds, twl, -1, ld, st, twload);
