@@ -383,11 +383,13 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
 // stage, clear and flush; 768 threads (three waves per SIMD, 156 registers)
 // measured best of 512, 768 and 1024 (which spills), and smaller tiles with
 // two or three workgroups per CU lose more to their halo.  FP64 takes two
-// waves per SIMD with a 12-byte spill.  At 256^3, FP32, one particle per cell:
-// 2.56 -> 1.8 ms, of which the LDS atomics are 0.5 ms and the global ones
-// 0.3 ms; FP64 at 128^3 with the reverse deposit 1.01 -> 0.77 ms.
-template <typename T, int TX, int TY, int TZ, int NT>
-__global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drift(PV<T> v, const T *__restrict__ phi, const T *__restrict__ chi,
+// waves per SIMD with a 12-byte spill, but one, without it, on grids of at
+// most one workgroup per CU (ONE; 32^3 with 6 per cell 128 -> 106 us).  At
+// 256^3, FP32, one particle per cell: 2.56 -> 1.8 ms, of which the LDS atomics
+// are 0.5 ms and the global ones 0.3 ms; FP64 at 128^3 with the reverse deposit
+// 1.01 -> 0.77 ms.
+template <typename T, int TX, int TY, int TZ, int NT, bool ONE>
+__global__ __launch_bounds__(NT, sizeof(T) == 8 && !ONE ? 2 : 1) void k_adj_gr_kick_drift(PV<T> v, const T *__restrict__ phi, const T *__restrict__ chi,
                                                           const T *__restrict__ Bi, T *lx, T *lq, T *lphi, T *lchi,
                                                           T *lB, int64_t M, AdjKD s)
 {
@@ -420,25 +422,45 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
     for (int e = tid; e < X2::END; e += NT) acc[e] = 0.0;
     int32_t rb0, incl;
     tile_rows_load<TX, TY, NROW>(v.start, N, x0, y0, z0, lane, rb0, incl);
-    const int maxrow = (int)wave_max_u32((uint32_t)incl);
+    __syncthreads();  // here, so that the wait for the rows' starts comes after it
+    // (the same in every lane; scalar, so that the walk below costs no vector registers)
+    const int maxrow = __builtin_amdgcn_readfirstlane((int)wave_max_u32((uint32_t)incl));
     incl = wave_row_scan(incl, lane);
-    const int total = __shfl(incl, NROW - 1, 64);
-    // A tile with a crowded row (64 or more particles in its 16 cells; a row of
-    // an unclustered state of one particle per cell reaches about 35) hands
-    // consecutive particles to different waves, so the field-adjoint atomics
-    // of one instruction rarely meet on one LDS address; other tiles keep
-    // consecutive particles in consecutive lanes, whose loads coalesce.
-    // 256^3 mixed states, both reverse kernels (measured before the loads were
-    // requested together): 4.07 and 3.16 ms (a tenth of the particles in
-    // clumps, none) against 4.38 and 3.13 ms with the line at 32, 4.05 and
-    // 3.16 ms at 100; 6.47, 6.65, 6.49 ms with four tenths in clumps
+    const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, NROW - 1, 64));
+    // The walk.  Consecutive particles in consecutive lanes coalesce their loads
+    // but meet on one LDS address when they share a cell; a spread tile's lanes
+    // take particles K NW apart (K passes of the tile's waves to a block).
+    // Grids of more than one workgroup per CU spread the tiles with a crowded
+    // row: 4 TX or more particles (a row of an unclustered state of one per
+    // cell reaches about half of that), K = 1, or four times the tile's mean
+    // row and TX more, a clump, with K by its excess.  Smaller grids live in
+    // the caches and spread from a quarter of a particle per cell on; with the
+    // small tile's few waves each lane takes one contiguous chunk (K = passes).
+    // Against K = 1 in every spread tile: FP64 32^3 with 1 / 2 / 6 per cell 29.1 /
+    // 60.1 / 234 -> 24.3 / 40.6 / 106 us, 64^3 with half of the particles in clumps
+    // 105 -> 81; FP32 64^3 with one per cell 55.6 -> 46.2 (0.3 and 0.4 of them in
+    // clumps 46.0 -> 33.8), 128^3 with 0.3, 0.9 of them in clumps 247 -> 191 us.
+    // Chunks everywhere lose where the grid fills the card: FP32 128^3, 6 per
+    // cell 3.45 against 2.89 ms, 256^3 with one per cell 2.35 against 1.82 ms.
     constexpr int NW = NT / 64;
-    const bool spread = maxrow >= 4 * TX;
-    const int niter = (total + NT - 1) / NT;  // the same for every lane of the workgroup
-    __syncthreads();
+    const int passes = (total + NT - 1) / NT, mean = total / NROW;
+    const bool clumped = maxrow >= 4 * mean + TX;
+    const bool spread = ONE ? 4 * total >= TX * TY * TZ : clumped || maxrow >= 4 * TX;
+    int K = 1, niter = passes;
+    if (spread && ((ONE && TX < 16) || clumped)) {
+        // the passes in blocks of K that are nearly full
+        const int want = ONE && TX < 16 ? passes : (maxrow - mean) / (2 * NW);
+        const int blocks = max(1, passes / max(1, min(want, 64)));
+        K = max(1, (passes + blocks - 1) / blocks);
+        niter = K * ((passes + K - 1) / K);
+    }
+    const int first = spread ? lane * (K * NW) + (tid >> 6) : tid;
+    const int jump = spread ? 64 * K * NW - (K - 1) * NW : NT;
     const int64_t n = v.n;
-    for (int it = 0; it < niter; it++) {
-        const int64_t p = tile_locate<NROW>(rb0, incl, it * NT + (spread ? lane * NW + (tid >> 6) : tid));
+    for (int it = 0, j = 0, at = 0; it < niter; it++) {
+        const int64_t p = tile_locate<NROW>(rb0, incl, first + at);
+        if (++j == K) { j = 0; at += jump; }
+        else at += NW;
         if (p < 0) continue;
         const int64_t id = v.id[p];
         int x, y, z;
@@ -448,7 +470,7 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
         const T qt[3] = {v.q0[p], v.q1[p], v.q2[p]};
         T LX[3], LQ[3], nx[3], nq[3];
 #pragma unroll
-        for (int j = 0; j < 3; j++) { LX[j] = lx[j * n + id]; LQ[j] = lq[j * n + id]; }
+        for (int i = 0; i < 3; i++) { LX[i] = lx[i * n + id]; LQ[i] = lq[i * n + id]; }
         const uint32_t cx = x & (TX - 1), cy = y & (TY - 1), cz = z & (TZ - 1);
         const BoxField<T, XP> Fp{fld, XP::corner(cx, cy, cz)};
         const BoxField<T, XC> Fc{fld, XC::corner(cx, cy, cz)};
@@ -462,7 +484,7 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 ? 2 : 1) void k_adj_gr_kick_drif
         };
         adj_gr_particle<T>(rt, qt, LX, LQ, Fp, Fc, F0, F1, F2, N, s, nx, nq, sc);
 #pragma unroll
-        for (int j = 0; j < 3; j++) { lx[j * n + id] = nx[j]; lq[j * n + id] = nq[j]; }
+        for (int i = 0; i < 3; i++) { lx[i * n + id] = nx[i]; lq[i * n + id] = nq[i]; }
     }
     __syncthreads();
     auto flush = [&](auto box, T *dst) {
@@ -842,31 +864,34 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
     const double bk = a_k * a_k * (double)c->N, bd = a_d * a_d * (double)c->N, K = dtau_k * c->N;
     AdjKD s{nf_k, nf_d, a_k, a_d, dtau_k, dtau_d, bk, bd, K, 1.0 / bk, 1.0 / bd, K / bk, dtau_d / bd};
     const int N = c->N;
-    auto launch = [&](auto tx, auto ty, auto tz, auto nt) {
+    auto launch = [&](auto tx, auto ty, auto tz, auto nt, auto one) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value, TZ = decltype(tz)::value;
         constexpr int NT = decltype(nt)::value;
         const unsigned nb = (unsigned)((int64_t)(N / TX) * (N / TY) * (N / TZ));
-        hipLaunchKernelGGL((k_adj_gr_kick_drift<T, TX, TY, TZ, NT>), dim3(nb), dim3(NT), 0, c->stream, make_pv<T>(p),
-                           phi, chi, Bi, lx, lq, lphi, lchi, lB, c->M, s);
+        hipLaunchKernelGGL((k_adj_gr_kick_drift<T, TX, TY, TZ, NT, decltype(one)::value>), dim3(nb), dim3(NT), 0,
+                           c->stream, make_pv<T>(p), phi, chi, Bi, lx, lq, lphi, lchi, lB, c->M, s);
     };
     using I4 = std::integral_constant<int, 4>;
     using I8 = std::integral_constant<int, 8>;
+    using I16 = std::integral_constant<int, 16>;
     using I256 = std::integral_constant<int, 256>;
+    // the grids of up to one workgroup per CU (256) take the kernel's ONE form
     if (p->n > 0) {
-        bool done = false;
         if constexpr (sizeof(T) == 4) {
             // FP64 fields and accumulators take the smaller tile, and so do
             // meshes whose large tiles would leave CUs idle (both reverse
             // kernels at 32^3: 57 against 94 us with 32 large tiles; at 64^3,
-            // 256 large tiles, 137 against 150 us)
-            if (N >= 64) {
-                launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 768>{});
-                done = true;
-            }
+            // 256 large tiles, 137 against 150 us).  512 threads on the small
+            // tile: 16^3 with 0.4 of 0.3 per cell in clumps 17.8 -> 14.2 us
+            using I768 = std::integral_constant<int, 768>;
+            if (N >= 128) launch(I16{}, I8{}, I8{}, I768{}, std::false_type{});
+            else if (N == 64) launch(I16{}, I8{}, I8{}, I768{}, std::true_type{});
+            else if (N >= 8) launch(I8{}, I8{}, I4{}, std::integral_constant<int, 512>{}, std::true_type{});
+        } else {
+            if (N >= 64) launch(I8{}, I8{}, I4{}, I256{}, std::false_type{});
+            else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{}, std::true_type{});
         }
-        if (done) {
-        } else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{});
-        else launch(I4{}, I4{}, I4{}, I256{});
+        if (N < 8) launch(I4{}, I4{}, I4{}, I256{}, std::true_type{});
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
