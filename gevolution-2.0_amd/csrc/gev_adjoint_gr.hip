@@ -387,8 +387,8 @@ __device__ __forceinline__ void adj_gr_particle(const T rt[3], const T qt[3], co
 // most one workgroup per CU (ONE; 32^3 with 6 per cell 128 -> 106 us).  At
 // 256^3, FP32, one particle per cell: 2.56 -> 1.8 ms, of which the LDS atomics
 // are 0.5 ms and the global ones 0.3 ms; FP64 at 128^3 with the reverse deposit
-// 1.01 -> 0.77 ms.
-template <typename T, int TX, int TY, int TZ, int NT, bool ONE>
+// 1.01 -> 0.77 ms.  R is the precision of the per-particle arithmetic.
+template <typename T, int TX, int TY, int TZ, int NT, bool ONE, typename R = T>
 __global__ __launch_bounds__(NT, sizeof(T) == 8 && !ONE ? 2 : 1) void k_adj_gr_kick_drift(PV<T> v, const T *__restrict__ phi, const T *__restrict__ chi,
                                                           const T *__restrict__ Bi, T *lx, T *lq, T *lphi, T *lchi,
                                                           T *lB, int64_t M, AdjKD s)
@@ -467,24 +467,24 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 && !ONE ? 2 : 1) void k_adj_gr_k
         cell_coords(v.cell[p], N, v.lg, x, y, z);
         T rt[3];
         ref_dist(v, p, x, y, z, rt);
-        const T qt[3] = {v.q0[p], v.q1[p], v.q2[p]};
-        T LX[3], LQ[3], nx[3], nq[3];
+        const R r[3] = {rt[0], rt[1], rt[2]}, q[3] = {v.q0[p], v.q1[p], v.q2[p]};
+        R LX[3], LQ[3], nx[3], nq[3];
 #pragma unroll
         for (int i = 0; i < 3; i++) { LX[i] = lx[i * n + id]; LQ[i] = lq[i * n + id]; }
         const uint32_t cx = x & (TX - 1), cy = y & (TY - 1), cz = z & (TZ - 1);
-        const BoxField<T, XP> Fp{fld, XP::corner(cx, cy, cz)};
-        const BoxField<T, XC> Fc{fld, XC::corner(cx, cy, cz)};
-        const BoxField<T, X0> F0{fld, X0::corner(cx, cy, cz)};
-        const BoxField<T, X1> F1{fld, X1::corner(cx, cy, cz)};
-        const BoxField<T, X2> F2{fld, X2::corner(cx, cy, cz)};
-        auto sc = [&](const auto &F, int dx, int dy, int dz, T val) {
+        const BoxField<T, XP, R> Fp{fld, XP::corner(cx, cy, cz)};
+        const BoxField<T, XC, R> Fc{fld, XC::corner(cx, cy, cz)};
+        const BoxField<T, X0, R> F0{fld, X0::corner(cx, cy, cz)};
+        const BoxField<T, X1, R> F1{fld, X1::corner(cx, cy, cz)};
+        const BoxField<T, X2, R> F2{fld, X2::corner(cx, cy, cz)};
+        auto sc = [&](const auto &F, int dx, int dy, int dz, R val) {
             using X = typename std::decay_t<decltype(F)>::Box;
             __hip_atomic_fetch_add(&acc[F.o + X::step(dx, dy, dz)], (double)val, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_WORKGROUP);
         };
-        adj_gr_particle<T>(rt, qt, LX, LQ, Fp, Fc, F0, F1, F2, N, s, nx, nq, sc);
+        adj_gr_particle<R>(r, q, LX, LQ, Fp, Fc, F0, F1, F2, N, s, nx, nq, sc);
 #pragma unroll
-        for (int i = 0; i < 3; i++) { lx[i * n + id] = nx[i]; lq[i * n + id] = nq[i]; }
+        for (int i = 0; i < 3; i++) { lx[i * n + id] = (T)nx[i]; lq[i * n + id] = (T)nq[i]; }
     }
     __syncthreads();
     auto flush = [&](auto box, T *dst) {
@@ -637,7 +637,7 @@ __device__ __forceinline__ void adj_gr_deposit_particle(const T rt[3], const T q
 // site at the end.  72 KB of LDS per FP32 tile allow two workgroups per CU:
 // with 512 threads each they fill four waves per SIMD (110 registers), with
 // 256 only two (256^3, one particle per cell: 1.26 -> 0.90 ms).
-template <typename T, int TX, int TY, int TZ, int NT>
+template <typename T, int TX, int TY, int TZ, int NT, typename R = T>
 __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restrict__ phi, const T *__restrict__ lT00,
                                                        const T *__restrict__ lTij, const T *__restrict__ lL, T *lx,
                                                        T *lq, T *lphi, int64_t M, double m00, double mij, double m0i,
@@ -699,22 +699,22 @@ __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restr
         cell_coords(v.cell[p], N, v.lg, x, y, z);
         T rt[3];
         ref_dist(v, p, x, y, z, rt);
-        const T qt[3] = {v.q0[p], v.q1[p], v.q2[p]};
-        T LX[3], LQ[3];
+        const R r[3] = {rt[0], rt[1], rt[2]}, q[3] = {v.q0[p], v.q1[p], v.q2[p]};
+        R LX[3], LQ[3];
 #pragma unroll
         for (int j = 0; j < 3; j++) { LX[j] = lx[j * n + id]; LQ[j] = lq[j * n + id]; }
         const int o = (x - x0) + SX * ((y - y0) + SY * (z - z0));
-        auto F = [&](int f, int dx, int dy, int dz) -> T { return fld[f][o + dx + SX * dy + SX * SY * dz]; };
-        auto sc = [&](int b, T val) {
+        auto F = [&](int f, int dx, int dy, int dz) -> R { return fld[f][o + dx + SX * dy + SX * SY * dz]; };
+        auto sc = [&](int b, R val) {
             __hip_atomic_fetch_add(&acc[o + ((b >> 2) & 1) + SX * ((b >> 1) & 1) + SX * SY * (b & 1)], (double)val,
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
         };
-        T gx[3], gq[3];
-        adj_gr_deposit_particle<T>(rt, qt, F, has_phi, has_links, N, m00, mij, m0i, a, gx, gq, sc);
+        R gx[3], gq[3];
+        adj_gr_deposit_particle<R>(r, q, F, has_phi, has_links, N, m00, mij, m0i, a, gx, gq, sc);
 #pragma unroll
         for (int j = 0; j < 3; j++) {
-            lx[j * n + id] = LX[j] + gx[j];
-            lq[j * n + id] = LQ[j] + gq[j];
+            lx[j * n + id] = (T)(LX[j] + gx[j]);
+            lq[j * n + id] = (T)(LQ[j] + gq[j]);
         }
     }
     if (out_phi) {
@@ -864,12 +864,12 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
     const double bk = a_k * a_k * (double)c->N, bd = a_d * a_d * (double)c->N, K = dtau_k * c->N;
     AdjKD s{nf_k, nf_d, a_k, a_d, dtau_k, dtau_d, bk, bd, K, 1.0 / bk, 1.0 / bd, K / bk, dtau_d / bd};
     const int N = c->N;
-    auto launch = [&](auto tx, auto ty, auto tz, auto nt, auto one) {
+    auto launch = [&](auto tx, auto ty, auto tz, auto nt, auto one, auto r) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value, TZ = decltype(tz)::value;
         constexpr int NT = decltype(nt)::value;
         const unsigned nb = (unsigned)((int64_t)(N / TX) * (N / TY) * (N / TZ));
-        hipLaunchKernelGGL((k_adj_gr_kick_drift<T, TX, TY, TZ, NT, decltype(one)::value>), dim3(nb), dim3(NT), 0,
-                           c->stream, make_pv<T>(p), phi, chi, Bi, lx, lq, lphi, lchi, lB, c->M, s);
+        hipLaunchKernelGGL((k_adj_gr_kick_drift<T, TX, TY, TZ, NT, decltype(one)::value, decltype(r)>), dim3(nb),
+                           dim3(NT), 0, c->stream, make_pv<T>(p), phi, chi, Bi, lx, lq, lphi, lchi, lB, c->M, s);
     };
     using I4 = std::integral_constant<int, 4>;
     using I8 = std::integral_constant<int, 8>;
@@ -882,16 +882,22 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
             // meshes whose large tiles would leave CUs idle (both reverse
             // kernels at 32^3: 57 against 94 us with 32 large tiles; at 64^3,
             // 256 large tiles, 137 against 150 us).  512 threads on the small
-            // tile: 16^3 with 0.4 of 0.3 per cell in clumps 17.8 -> 14.2 us
+            // tile: 16^3 with 0.4 of 0.3 per cell in clumps 17.8 -> 14.2 us.
+            // The small tiles of 16^3 and 32^3 add 3.3 FP32 partial sums at a
+            // site where large ones would add 2.3; FP64 arithmetic more than
+            // makes up for it (rms errors against FP64 at 32^3: lx 0.9 -> 0.3e-7,
+            // phi 1.6 -> 0.4e-7, B 0.67 -> 0.33e-7; one per cell 19.7 -> 21.7 us
+            // of 39.4 with large tiles in FP32)
             using I768 = std::integral_constant<int, 768>;
-            if (N >= 128) launch(I16{}, I8{}, I8{}, I768{}, std::false_type{});
-            else if (N == 64) launch(I16{}, I8{}, I8{}, I768{}, std::true_type{});
-            else if (N >= 8) launch(I8{}, I8{}, I4{}, std::integral_constant<int, 512>{}, std::true_type{});
+            if (N >= 128) launch(I16{}, I8{}, I8{}, I768{}, std::false_type{}, T());
+            else if (N == 64) launch(I16{}, I8{}, I8{}, I768{}, std::true_type{}, T());
+            else if (N >= 16) launch(I8{}, I8{}, I4{}, std::integral_constant<int, 512>{}, std::true_type{}, 0.0);
+            else if (N >= 8) launch(I8{}, I8{}, I4{}, std::integral_constant<int, 512>{}, std::true_type{}, T());
         } else {
-            if (N >= 64) launch(I8{}, I8{}, I4{}, I256{}, std::false_type{});
-            else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{}, std::true_type{});
+            if (N >= 64) launch(I8{}, I8{}, I4{}, I256{}, std::false_type{}, T());
+            else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{}, std::true_type{}, T());
         }
-        if (N < 8) launch(I4{}, I4{}, I4{}, I256{}, std::true_type{});
+        if (N < 8) launch(I4{}, I4{}, I4{}, I256{}, std::true_type{}, T());
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;
@@ -904,26 +910,23 @@ int adj_gr_deposit_impl(gev_pcls *p, const T *phi, const T *lT00, const T *lTij,
     gev_ctx *c = p->ctx;
     const double dx = 1.0 / (double)c->N, m = p->mass / (dx * dx * dx);
     const int N = c->N;
-    auto launch = [&](auto tx, auto ty, auto tz, auto nt) {
+    auto launch = [&](auto tx, auto ty, auto tz, auto nt, auto r) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value, TZ = decltype(tz)::value;
         constexpr int NT = decltype(nt)::value;
         const unsigned nb = (unsigned)((int64_t)(N / TX) * (N / TY) * (N / TZ));
-        hipLaunchKernelGGL((k_adj_gr_deposit<T, TX, TY, TZ, NT>), dim3(nb), dim3(NT), 0, c->stream, make_pv<T>(p), phi,
+        hipLaunchKernelGGL((k_adj_gr_deposit<T, TX, TY, TZ, NT, decltype(r)>), dim3(nb), dim3(NT), 0, c->stream, make_pv<T>(p), phi,
                            lT00, lTij, lL, lx, lq, lphi, c->M, phi ? m / a : m, tij_scale * m / a, m, a);
     };
     using I4 = std::integral_constant<int, 4>;
     using I8 = std::integral_constant<int, 8>;
+    using I256 = std::integral_constant<int, 256>;
     if (p->n > 0) {
-        bool done = false;
-        if constexpr (sizeof(T) == 4) {  // FP64 fields take twice the LDS: the smaller tile; N as above
-            if (N >= 64) {
-                launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 512>{});
-                done = true;
-            }
-        }
-        if (done) {
-        } else if (N >= 8) launch(I8{}, I8{}, I4{}, std::integral_constant<int, 256>{});
-        else launch(I4{}, I4{}, I4{}, std::integral_constant<int, 256>{});
+        if constexpr (sizeof(T) == 4) {  // tiles, and FP64 arithmetic, by the same rules as above
+            if (N >= 64) launch(std::integral_constant<int, 16>{}, I8{}, I8{}, std::integral_constant<int, 512>{}, T());
+            else if (N >= 16) launch(I8{}, I8{}, I4{}, I256{}, 0.0);
+            else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{}, T());
+        } else if (N >= 8) launch(I8{}, I8{}, I4{}, I256{}, T());
+        if (N < 8) launch(I4{}, I4{}, I4{}, I256{}, T());
     }
     GEV_HIP(hipGetLastError());
     return GEV_OK;

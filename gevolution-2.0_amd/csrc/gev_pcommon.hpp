@@ -215,11 +215,11 @@ __device__ __forceinline__ void box_put(T *lds, const std::array<T, K> &t)
         if (e < X::N) lds[X::END - X::N + e] = t[k];
     }
 }
-template <typename T, class X> struct BoxField {
+template <typename T, class X, typename R = T> struct BoxField {
     using Box = X;
     const T *lds;
     uint32_t o;  // X::corner of the particle's cell
-    __device__ __forceinline__ T operator()(int dx, int dy, int dz) const { return lds[o + X::step(dx, dy, dz)]; }
+    __device__ __forceinline__ R operator()(int dx, int dy, int dz) const { return (R)lds[o + X::step(dx, dy, dz)]; }
 };
 
 // reciprocal and square roots: FP32 uses the hardware approximations (1 ulp),
