@@ -195,6 +195,10 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
         if (lane >= o) incl += y;
     }
     if (lane == 63) wsum[wv] = incl;
+    if constexpr (MASS) {
+        const uint32_t fullest = wave_max_u32((uint32_t)len);
+        if (lane == 0) wpm[wv] = fullest;
+    }
     __syncthreads();
     int32_t off = 0;
     for (int j = 0; j < wv; j++) off += wsum[j];
@@ -307,6 +311,21 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
     // measured slower with it)
     const bool chunk = sizeof(T) == 4 && U == 1 && DEP_CHUNK_X4 > 0 && 4 * total >= DEP_CHUNK_X4 * NCELL;
     const int32_t Q = (total + 63) / 64;
+    // MASS: a tile with a clump, a halo row 24 particles or more above the mean
+    // row, walks the corners in an order by lane (below): 64-bit atomics on one
+    // LDS address cost more than 32-bit ones, and clumped states lost what the
+    // long rows give (256^3 with 0.45 per cell, 0.4 and 0.9 of them in clumps: 16x8x8
+    // tiles 98 and 135 us, these without that order 108 and 154, with it 73 and
+    // 83; 512^3 847 and 1047, 811 and 1138, 576 and 628).  Lines at 12 and 40
+    // measured the same and up to 10 % slower; in tiles without a clump the order
+    // itself costs (256^3, 0.1 per cell, unclumped 31 -> 36 us).
+    bool clump = false;
+    if constexpr (MASS) {
+        uint32_t fullest = 0;
+#pragma unroll
+        for (int j = 0; j < NW; j++) fullest = max(fullest, wpm[j]);
+        clump = (int32_t)fullest >= total / NR + 24;
+    }
     for (int32_t i0 = 0; i0 < total; i0 += U * PT_NT) {
         int run[U];
         int64_t pu[U];
@@ -411,6 +430,25 @@ __global__ __launch_bounds__(PT_NT) void k_deposit(PV<T> v, T *out, T *out2, T *
                 }
             } else {
                 const T sc = MASS ? (T)1073741824 : (FIX ? (T)S0 : o);
+                if (MASS && clump) {
+                    // consecutive lanes start at different corners of their
+                    // cells (each axis walked up or down by a bit of the lane),
+                    // so the members of one cell meet an eighth as often on one
+                    // LDS address: the same products and the same integer sums
+                    const bool fx = lane & 1, fy = lane & 2, fz = lane & 4;
+                    const T wx[2] = {fx ? rd[0] : ox, fx ? ox : rd[0]}, wy[2] = {fy ? rd[1] : oy, fy ? oy : rd[1]},
+                            wz[2] = {fz ? rd[2] : oz, fz ? oz : rd[2]};
+                    const bool ix[2] = {fx ? inx1 : inx0, fx ? inx0 : inx1}, iy[2] = {fy ? iny1 : iny0, fy ? iny0 : iny1},
+                               iz[2] = {fz ? inz1 : inz0, fz ? inz0 : inz1};
+                    const int dx = fx ? -1 : 1, dy = fy ? -TX : TX, dz = fz ? -TX * TY : TX * TY;
+                    const int s0 = sb + (fx ? 1 : 0) + (fy ? TX : 0) + (fz ? TX * TY : 0);
+#pragma unroll
+                    for (int b = 0; b < 8; b++) {
+                        const int bx = (b >> 2) & 1, by = (b >> 1) & 1, bz = b & 1;
+                        if (ix[bx] && iy[by] && iz[bz])
+                            lds_add(&acc[0][s0 + bx * dx + by * dy + bz * dz], sc * (wx[bx] * (wy[by] * wz[bz])));
+                    }
+                } else
 #pragma unroll
                 for (int b = 0; b < 8; b++) {
                     const int bx = (b >> 2) & 1, by = (b >> 1) & 1, bz = b & 1;
