@@ -112,7 +112,7 @@ __device__ __forceinline__ void pgrad_matrix(const F0 &B0, const F1 &B1, const F
 // N, 1 / bc_k, 1 / bc_d, K / bc_k and dtau_d / bc_d
 struct AdjKD {
     int nf_k, nf_d;
-    double a_k, a_d, dtau_k, dtau_d, bc_k, bc_d, K, ibk, ibd, K_bk, d_bd;
+    double a_k, a_d, dtau_d, K, ibk, ibd, K_bk, d_bd;
 };
 
 // Reverse of the fused kick + drift of one particle (state before the kick),
@@ -862,7 +862,7 @@ int adj_gr_kick_drift_impl(gev_pcls *p, const T *phi, const T *chi, const T *Bi,
 {
     gev_ctx *c = p->ctx;
     const double bk = a_k * a_k * (double)c->N, bd = a_d * a_d * (double)c->N, K = dtau_k * c->N;
-    AdjKD s{nf_k, nf_d, a_k, a_d, dtau_k, dtau_d, bk, bd, K, 1.0 / bk, 1.0 / bd, K / bk, dtau_d / bd};
+    AdjKD s{nf_k, nf_d, a_k, a_d, dtau_d, K, 1.0 / bk, 1.0 / bd, K / bk, dtau_d / bd};
     const int N = c->N;
     auto launch = [&](auto tx, auto ty, auto tz, auto nt, auto one, auto r) {
         constexpr int TX = decltype(tx)::value, TY = decltype(ty)::value, TZ = decltype(tz)::value;

@@ -414,10 +414,11 @@ __global__ __launch_bounds__(NL * N / 16) void k_r2c_x_multi(Src src, cx<T> *__r
 // the diagonal and the three off-diagonal components carry it:
 //   0: S_xx - S_zz, 1: S_yy - S_zz, 2: S_xy, 3: S_xz, 4: S_yz
 // (five half spectra to write, transform and read instead of six: 512^3 FP64
-// phi + chi + B solves 20.48 -> 19.82 ms).  FP64 only: in FP32 the six
-// components as they are gain less (1 % of a 512^3 cycle) than what keeping
-// the mixed form's chi unchanged to the last bit is worth, since particles at
-// a cell face move their link deposits by a whole site on a last-bit change.
+// phi + chi + B solves 20.48 -> 19.82 ms).  FP64 only.  In FP32 five gain 1 % of
+// a 512^3 mixed cycle (meshes of 256^3 and more; smaller ones transform planes);
+// six keep that cycle's chi as it is, where a last-bit change lets some particle
+// cross a cell face a cycle earlier or later and moves its link deposits by a
+// site (largest change of B 2e-3 to 3e-3, as between two runs of one build).
 template <typename T> constexpr int sij_spectra() { return sizeof(T) == 8 ? 5 : 6; }
 // From prepareFTsource(phi, Tij, coeff), Tij's component c at Tij + c M:
 template <typename T, int N> struct SrcSijX {
@@ -1162,11 +1163,11 @@ template <typename T, int N, class S> struct SrcPut : S {
 
 template <typename T, int N> struct CompT00 {
     SrcT00<T, N> s;
-    T *put;  // the source, written back for N < 128
+    T *put;  // the source, written back
     template <class F> __device__ __forceinline__ void with(int, F f) const
     {
-        if constexpr (N < 128) f(SrcPut<T, N, SrcT00<T, N>>(s, put));
-        else f(s);
+        static_assert(N < 128, "the T00 source is formed in planes up to 64^3 only");
+        f(SrcPut<T, N, SrcT00<T, N>>(s, put));
     }
 };
 
