@@ -219,8 +219,8 @@ class PMRunGR:
 
     def _fields(self, k, phi_old, chi_old):
         """the cycle's deposits and metric solves from the container's state;
-        returns (phi, chi, B) of the cycle (new tensors) and fills self.T00,
-        self.Tij, self.L"""
+        returns (phi, chi, B) of the cycle (new tensors) and fills self.T00 and
+        self.L; self.Tij holds Tij, below N = 128 the Sij formed from it"""
         s, c, p, k_ = self.sched[k], self.ctx, self.pcls, self._coef(k)
         p.project_T00_Tij_T0i_links(self.T00, self.Tij, self.L, a=s["a"], phi=phi_old, coeff=1.0)
         # T00 and the links stay as they are for the reverse cycle: the phi
