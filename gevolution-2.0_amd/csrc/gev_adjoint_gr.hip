@@ -429,19 +429,21 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 && !ONE ? 2 : 1) void k_adj_gr_k
     const int total = __builtin_amdgcn_readfirstlane(__shfl(incl, NROW - 1, 64));
     // The walk.  Consecutive particles in consecutive lanes coalesce their loads
     // but meet on one LDS address when they share a cell; a spread tile's lanes
-    // take particles K NW apart (K passes of the tile's waves to a block).
-    // Grids of more than one workgroup per CU spread the tiles with a crowded
-    // row: 4 TX or more particles (a row of an unclustered state of one per
-    // cell reaches about half of that), K = 1, or four times the tile's mean
-    // row and TX more, a clump, with K by its excess.  Smaller grids live in
-    // the caches and spread from a quarter of a particle per cell on; with the
+    // take particles K NW apart (K passes of the tile's waves to a block). Grids
+    // of more than one workgroup per CU spread the tiles with a crowded row: 4 TX
+    // or more particles (a row of an unclustered state of one per cell reaches
+    // about half of that), K = 1, or four times the tile's mean row and TX more, a
+    // clump, with K by a quarter of its excess (half of it: 256^3 one per cell, a
+    // tenth and half of them in clumps, 0.5 and 1.3 % slower; with the line at six
+    // times the mean FP64 64^3, half in clumps, 80 -> 104 us).  Smaller grids live
+    // in the caches and spread from a quarter of a particle per cell on; with the
     // small tile's few waves each lane takes one contiguous chunk (K = passes).
     // Against K = 1 in every spread tile: FP64 32^3 with 1 / 2 / 6 per cell 29.1 /
-    // 60.1 / 234 -> 24.3 / 40.6 / 106 us, 64^3 with half of the particles in clumps
-    // 105 -> 81; FP32 64^3 with one per cell 55.6 -> 46.2 (0.3 and 0.4 of them in
-    // clumps 46.0 -> 33.8), 128^3 with 0.3, 0.9 of them in clumps 247 -> 191 us.
-    // Chunks everywhere lose where the grid fills the card: FP32 128^3, 6 per
-    // cell 3.45 against 2.89 ms, 256^3 with one per cell 2.35 against 1.82 ms.
+    // 60.1 / 234 -> 24.3 / 40.6 / 106 us, 64^3 with half of the particles in
+    // clumps 105 -> 80; FP32 64^3 with one per cell 55.3 -> 46.4 (0.3 and 0.4 of
+    // them in clumps 46.0 -> 36.0), 128^3 with 0.3, 0.9 of them in clumps 247 ->
+    // 191 us. Chunks everywhere lose where the grid fills the card: FP32 128^3, 6
+    // per cell 3.45 against 2.89 ms, 256^3 with one per cell 2.35 against 1.82 ms.
     constexpr int NW = NT / 64;
     const int passes = (total + NT - 1) / NT, mean = total / NROW;
     const bool clumped = maxrow >= 4 * mean + TX;
@@ -449,7 +451,7 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 && !ONE ? 2 : 1) void k_adj_gr_k
     int K = 1, niter = passes;
     if (spread && ((ONE && TX < 16) || clumped)) {
         // the passes in blocks of K that are nearly full
-        const int want = ONE && TX < 16 ? passes : (maxrow - mean) / (2 * NW);
+        const int want = ONE && TX < 16 ? passes : (maxrow - mean) / (4 * NW);
         const int blocks = max(1, passes / max(1, min(want, 64)));
         K = max(1, (passes + blocks - 1) / blocks);
         niter = K * ((passes + K - 1) / K);
@@ -658,7 +660,10 @@ __global__ __launch_bounds__(NT) void k_adj_gr_deposit(PV<T> v, const T *__restr
         // physics instead of after it.  Both reverse kernels: 256^3 mixed 3.86
         // -> 3.73 ms (IDs in no order 8.25 -> 7.87), 128^3 FP64 754 -> 730 us,
         // 64^3 mixed 91 -> 84 us (IDs in no order 142 -> 146); the old adjoints
-        // alone 3.76 ms, 757 and 86 us
+        // alone 3.76 ms, 757 and 86 us.  128^3 mixed loses with them and with 512
+        // threads where IDs are in no order or particles few: 0.3 per cell 149 ->
+        // 160 us, 155 with the old adjoints late, which cost 64^3 5-13 % and 32^3
+        // 3-25 %.
         constexpr int NI = (NS + NT - 1) / NT;
         T ld[NI][11];
 #pragma unroll
