@@ -456,11 +456,13 @@ __global__ __launch_bounds__(NT, sizeof(T) == 8 && !ONE ? 2 : 1) void k_adj_gr_k
         K = max(1, (passes + blocks - 1) / blocks);
         niter = K * ((passes + K - 1) / K);
     }
-    const int first = spread ? lane * (K * NW) + (tid >> 6) : tid;
-    const int jump = spread ? 64 * K * NW - (K - 1) * NW : NT;
+    const uint32_t first = spread ? lane * (K * NW) + (tid >> 6) : tid;
+    const uint32_t jump = spread ? 64 * K * NW - (K - 1) * NW : NT;
     const int64_t n = v.n;
-    for (int it = 0, j = 0, at = 0; it < niter; it++) {
-        const int64_t p = tile_locate<NROW>(rb0, incl, first + at);
+    uint32_t at = 0;
+    for (int it = 0, j = 0; it < niter; it++) {
+        // (the last block may end up to 64 passes beyond the tile's particles)
+        const int64_t p = tile_locate<NROW>(rb0, incl, (int)min(first + at, (uint32_t)total));
         if (++j == K) { j = 0; at += jump; }
         else at += NW;
         if (p < 0) continue;
