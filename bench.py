@@ -225,7 +225,7 @@ def main():
         "config": {"workload": f"GR weak-field PM cycle (main.cu order), {N}^3 particles on {N}^3 mesh, "
                                f"L={L:g} Mpc/h, BBKS Zel'dovich IC z={args.z_in:g}, {total} cycles to "
                                f"z={args.z_end:g}, mixed precision (FP32 fields/FFT/deposit, FP64 k=0, "
-                               "chi combination, sums)",
+                               "chi sum over the kz groups, global sums)",
                    "mesh": N, "particles": N ** 3, "boxsize_mpc_h": L, "cycles": total,
                    "timed_cycles": win_m["timed_cycles"], "timed_z": win_m["timed_z"]},
         "all_cycles": win_m["all_cycles"],
@@ -291,7 +291,7 @@ def rows_next(cm, pm, fm, st, dtau, L, om, ol, fpg):
 # cycle (R = 4-byte reals, n particles, M cells): each input read once, each
 # output written once, no halo or re-read counted.
 def _bytes_models(M, n, R=4, links=True):
-    # links: the GR step sums T0i on the links in the T00+Tij pass (128 <= N <= 1024)
+    # links: the GR step sums T0i on the links in the T00+Tij pass (16 <= N <= 1024)
     nc = 10 if links else 7
     return {
         "kick_drift": (n * (7 * R + 8 * R + 8) + M * 5 * R,

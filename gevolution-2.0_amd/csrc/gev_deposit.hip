@@ -24,6 +24,7 @@
 // kinetic to rest energy) and scales so that bound is 2^30.  |q| is bounded
 // by the largest |q|^2 per 8^3-cell block that the last particle update
 // recorded (gev_pcls::qbound), or else by a pass over the tile's particles.
+// The mass deposit of sparse FP32 meshes sums in 64 bits at a fixed scale (DepRow).
 #include "gev_common.hpp"
 #include "gev_kernels.hpp"
 #include "gev_pcommon.hpp"

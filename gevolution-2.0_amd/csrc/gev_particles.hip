@@ -3,17 +3,18 @@
 //     positions in, FP64 or FP32 cell offsets plus an int32 cell key inside);
 //   * re-binning by cell: k_count ranks each particle in its cell with one
 //     counter atomic (the fused kick/drift in gev_pupdate.hip takes the same
-//     ranks itself), a three-kernel exclusive scan turns the counts into
-//     cell_start and clears the counters, k_perm writes each particle's old
-//     slot and cell key at its new slot, and k_gather copies the rest of the
-//     particle into the ping-pong arrays with coalesced stores;
+//     ranks itself), an exclusive scan (three kernels, two up to 128^3, one up
+//     to 16^3) turns the counts into cell_start and clears the counters, k_perm
+//     writes each particle's old slot and cell key at its new slot, and
+//     k_gather copies the rest of the particle into the ping-pong arrays with
+//     coalesced stores; below 2^20 particles k_scatter moves them in one pass;
 //   * the IC displacement and velocity gathers (one thread per particle in
 //     cell order).
 // The order of particles inside a cell follows the counter atomics, so it can
 // change from run to run; IDs, cell keys and cell_start do not.  The CIC
 // deposits live in gev_deposit.hip (LDS atomics: the FP64 sums are not
-// bit-reproducible from run to run, the FP32 form's 32-bit fixed-point sums
-// are) and the kick/drift in gev_pupdate.hip.
+// bit-reproducible from run to run, the FP32 form's fixed-point sums are) and
+// the kick/drift in gev_pupdate.hip.
 #include "gev_common.hpp"
 #include "gev_kernels.hpp"
 #include "gev_pcommon.hpp"

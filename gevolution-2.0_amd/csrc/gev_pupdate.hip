@@ -1,7 +1,8 @@
 // gev_pupdate.hip -- tiled particle updates (kick, drift, and both fused).
 //
 // One workgroup owns a tile of TX x TY x TZ cells.  Every field value the
-// update_q / update_pos stencils can touch (offsets -1..+2 around the tile)
+// update_q / update_pos stencils can touch (per field: phi at offsets -1..+2
+// around the tile, chi 0..1, B_i -1..1 along i and 0..1 across; KickBoxes)
 // is staged in LDS once; the tile's particles -- TY*TZ contiguous row
 // segments of the cell-sorted container -- are then spread over the threads
 // and read their ~60 stencil values from LDS instead of global memory.  The
@@ -308,7 +309,7 @@ template <typename T> static int launch_update(gev_pcls *p, const UpdParams &u, 
     }
     unsigned long long *slot = (unsigned long long *)(c->red + 8);
     const T *B0 = Bi, *B1 = Bi ? Bi + c->M : nullptr, *B2 = Bi ? Bi + 2 * c->M : nullptr;
-    // FP32 fits the 16x8x8 tile (5 staged fields, 46 KB of LDS); FP64 keeps 8x8x4
+    // FP32 fits the 16x8x8 tile (8194 staged values, 33 KB of LDS); FP64 keeps 8x8x4
     bool big = false;
     if constexpr (sizeof(T) == 4) big = N >= 16;
     if (big) {
